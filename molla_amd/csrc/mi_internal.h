@@ -255,6 +255,14 @@ int launch_attend(hipStream_t s, const float* q, int64_t q_stride, const uint16_
                   int32_t max_count, int32_t tokens, float* out, void* xq_out, void* work,
                   int32_t form = MI_CACHE_F16, const int32_t* kv_index = nullptr, int64_t index_stride = 0,
                   void* hx_out = nullptr);
+// One sequence's chunk of more than kMaxTokens tokens at head widths 64 and
+// 128, either cache form (attend_flash.hip); cache rows from the sequence's
+// start or through kv_index.  part_acc / part_ml as launch_attend carves them.
+bool flash_fits(int32_t heads, int32_t kv_heads, int32_t head_dim, int32_t tokens);
+int launch_attend_flash(hipStream_t s, const float* q, int64_t q_stride, const uint16_t* k_cache,
+                        const uint16_t* v_cache, int32_t heads, int32_t kv_heads, int32_t head_dim, float scale,
+                        const int32_t* pos, int32_t max_count, int32_t tokens, float* out, float* part_acc,
+                        float* part_ml, int32_t form, const int32_t* kv_index);
 int launch_argmax(hipStream_t s, const float* x, int32_t n, int32_t tokens, int32_t* out);
 size_t argmax_workspace(int32_t n, int32_t tokens);
 int launch_argmax_ws(hipStream_t s, const float* x, int32_t n, int32_t tokens, int32_t* out, void* work,

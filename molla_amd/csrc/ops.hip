@@ -479,21 +479,6 @@ __global__ __launch_bounds__(kAttnThreads) void attend_split_kernel(
   }
 }
 
-// A prefill chunk's attention slice on the matrix cores
-// (v_mfma_f32_16x16x32_f16): one block = one 64-key slice x one key head x
-// 64 query rows, the rows being TQ = 64 / GROUP consecutive tokens times the
-// GROUP query heads of that key head (row r = token r / GROUP, head r %
-// GROUP).  One sequence's chunk only (its tokens share the cache).
-//   S = Q K^T: queries as three halves (q1 = f16(q), q2 = f16(q - q1),
-//   q3 = f16(q - q1 - q2): every bit of the f32 query), keys exact halves,
-//   f32 accumulation.  Two halves (22 bits) were not enough: a softmax feels
-//   a score's absolute error, and scores of a few hundred turned the last
-//   bits of the query into 1e-4 of the output.
-//   P = exp(S*scale - rowmax) per row over the slice's live keys (key <
-//   pos[t] + 1, cell held), written as (m, l) like the VALU kernel.
-//   O = P V with P as two halves and V (staged transposed) exact halves.
-// The partial sums land where attend_split_kernel writes them, so
-// attend_merge_kernel folds them unchanged.
 // MFMA fragments (16x16x32): lane l holds row/column l % 16 and values
 // 8 (l / 16) .. +8 of the 32; the result element i of lane l is row
 // 4 (l / 16) + i, column l % 16.
@@ -504,183 +489,10 @@ __device__ __forceinline__ att_f4 att_mfma(att_h8 a, att_h8 b, att_f4 c) {
   return __builtin_amdgcn_mfma_f32_16x16x32_f16(a, b, c, 0, 0, 0);
 }
 
-constexpr int kChunkKeys = 64;
-// The matrix-core slices split P (at most 1) into two halves after lifting
+// The matrix-core slice splits P (at most 1) into two halves after lifting
 // it by 2^14, and scale the sums back: exact powers of two, which keep the
 // low halves of weights down to ~1e-8 out of the f16 subnormals.
 constexpr float kPLift = 16384.0f, kPDrop = 1.0f / 16384.0f;
-__host__ __device__ __forceinline__ int attn_chunk_pad(int d) { return d + 8; }  // halves per LDS row
-__host__ __device__ __forceinline__ size_t attn_chunk_lds_bytes(int head_dim) {
-  const int dp = attn_chunk_pad(head_dim), kp = kChunkKeys + 8;
-  return 2 * ((size_t)kChunkKeys * dp + (size_t)head_dim * kp + (size_t)2 * 4 * 16 * kp);
-}
-
-template <int GROUP, int D>
-__global__ __launch_bounds__(256) void attend_chunk_kernel(
-    const float* __restrict__ q, int64_t q_stride, const __half* __restrict__ kc, const __half* __restrict__ vc,
-    int heads, int kv_heads, float scale, const int32_t* __restrict__ pos_dev, int max_chunks,
-    float* __restrict__ part_acc, float* __restrict__ part_ml, const int32_t* __restrict__ kv_index, int tokens) {
-  constexpr int TQ = 64 / GROUP;
-  constexpr int DP = D + 8, KP = kChunkKeys + 8;
-  const int c = blockIdx.x, kvh = blockIdx.y, t0 = blockIdx.z * TQ;
-  const int t1 = min(t0 + TQ, tokens);
-  int count_max = 0;
-  for (int t = t0; t < t1; t++) count_max = max(count_max, pos_dev[t] + 1);
-  const int start = c * kChunkKeys;
-  if (start >= count_max) return;
-  const int nk_max = min(kChunkKeys, count_max - start);
-  const int kvw = kv_heads * D;
-  extern __shared__ uint4 lds4[];
-  _Float16* Ks = (_Float16*)lds4;
-  _Float16* Vt = Ks + kChunkKeys * DP;
-  _Float16* Ph = Vt + D * KP;
-  _Float16* Pl = Ph + 4 * 16 * KP;
-  const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
-  const int lm = lane & 15, lk = lane >> 4;
-
-  // keys (rows) and values (transposed); keys past the end repeat the last
-  // live one (masked below); every load issued before any LDS store
-  const __half* kbase = kc + (int64_t)kvh * D;
-  const __half* vbase = vc + (int64_t)kvh * D;
-  constexpr int pieces = D / 8, total = kChunkKeys * pieces, per = total / 256;
-  static_assert(total % 256 == 0, "whole pieces per thread");
-  uint4 kv[per], vv[per];
-#pragma unroll
-  for (int j = 0; j < per; j++) {
-    const int i = tid + j * 256;
-    const int key = min(i / pieces, nk_max - 1), pc = i % pieces;
-    const int cell = max(kv_cell(kv_index, 0, t0, start + key), 0);
-    const int64_t off = (int64_t)cell * kvw + pc * 8;
-    kv[j] = *(const uint4*)(kbase + off);
-    vv[j] = *(const uint4*)(vbase + off);
-  }
-  // this wave's 16 query rows straight into A fragments (row r = token
-  // t0 + r / GROUP, head kvh * GROUP + r % GROUP): lane row lm, values
-  // 32 ks + 8 lk .. +8 of each 32-value step, as three halves
-  const int row0 = wave * 16;
-  float4 qraw[D / 32][2];
-  {
-    const int r = row0 + lm, t = t0 + r / GROUP;
-    const float* qr = q + (int64_t)min(t, tokens - 1) * q_stride + (int64_t)(kvh * GROUP + r % GROUP) * D;
-#pragma unroll
-    for (int ks = 0; ks < D / 32; ks++) {
-      qraw[ks][0] = t < tokens ? *(const float4*)(qr + 32 * ks + 8 * lk) : make_float4(0.0f, 0.0f, 0.0f, 0.0f);
-      qraw[ks][1] = t < tokens ? *(const float4*)(qr + 32 * ks + 8 * lk + 4) : make_float4(0.0f, 0.0f, 0.0f, 0.0f);
-    }
-  }
-#pragma unroll
-  for (int j = 0; j < per; j++) {
-    const int i = tid + j * 256;
-    const int key = i / pieces, pc = i % pieces;
-    *(uint4*)(Ks + key * DP + pc * 8) = kv[j];
-    const _Float16* v8 = (const _Float16*)&vv[j];
-#pragma unroll
-    for (int d = 0; d < 8; d++) Vt[(pc * 8 + d) * KP + key] = v8[d];
-  }
-  __syncthreads();
-
-  // S for this wave's 16 rows x 64 keys
-  att_f4 sacc[4];
-#pragma unroll
-  for (int nt = 0; nt < 4; nt++) sacc[nt] = att_f4{0.0f, 0.0f, 0.0f, 0.0f};
-#pragma unroll
-  for (int ks = 0; ks < D / 32; ks++) {
-    att_h8 ah, am, al;
-    const float qf[8] = {qraw[ks][0].x, qraw[ks][0].y, qraw[ks][0].z, qraw[ks][0].w,
-                         qraw[ks][1].x, qraw[ks][1].y, qraw[ks][1].z, qraw[ks][1].w};
-#pragma unroll
-    for (int u = 0; u < 8; u++) {
-      const _Float16 h = (_Float16)qf[u];
-      const float r1 = qf[u] - (float)h;  // exact
-      const _Float16 mid = (_Float16)r1;
-      ah[u] = h;
-      am[u] = mid;
-      al[u] = (_Float16)(r1 - (float)mid);
-    }
-#pragma unroll
-    for (int nt = 0; nt < 4; nt++) {
-      const att_h8 b = *(const att_h8*)(Ks + (16 * nt + lm) * DP + 32 * ks + 8 * lk);
-      sacc[nt] = att_mfma(ah, b, sacc[nt]);
-      sacc[nt] = att_mfma(am, b, sacc[nt]);
-      sacc[nt] = att_mfma(al, b, sacc[nt]);
-    }
-  }
-  // rows 4 lk + i of this wave: token, its count, the slice's live keys
-  float mrow[4], lrow[4];
-  int cnt[4];
-  bool rowlive[4];
-#pragma unroll
-  for (int i = 0; i < 4; i++) {
-    const int r = row0 + 4 * lk + i, t = t0 + r / GROUP;
-    rowlive[i] = t < tokens;
-    cnt[i] = rowlive[i] ? pos_dev[t] + 1 : 0;
-    rowlive[i] = rowlive[i] && start < cnt[i];
-  }
-  float pv[4][4];
-#pragma unroll
-  for (int i = 0; i < 4; i++) {
-    float m = -INFINITY;
-#pragma unroll
-    for (int nt = 0; nt < 4; nt++) {
-      const int key = start + 16 * nt + lm;
-      const bool live = key < cnt[i] && (!kv_index || kv_cell(kv_index, 0, t0, key) >= 0);
-      pv[i][nt] = live ? sacc[nt][i] * scale : -INFINITY;
-      m = fmaxf(m, pv[i][nt]);
-    }
-#pragma unroll
-    for (int o = 8; o >= 1; o >>= 1) m = fmaxf(m, __shfl_xor(m, o));
-    float l = 0.0f;
-#pragma unroll
-    for (int nt = 0; nt < 4; nt++) {
-      pv[i][nt] = pv[i][nt] == -INFINITY ? 0.0f : expf(pv[i][nt] - m);
-      l += pv[i][nt];
-    }
-#pragma unroll
-    for (int o = 8; o >= 1; o >>= 1) l += __shfl_xor(l, o);
-    mrow[i] = m;
-    lrow[i] = l;
-  }
-  // P into this wave's LDS rows (hi and lo halves), read back as A fragments
-  _Float16* ph = Ph + wave * 16 * KP;
-  _Float16* pl = Pl + wave * 16 * KP;
-#pragma unroll
-  for (int i = 0; i < 4; i++)
-#pragma unroll
-    for (int nt = 0; nt < 4; nt++) {
-      const float p = pv[i][nt] * kPLift;  // see kPLift
-      const _Float16 h = (_Float16)p;
-      ph[(4 * lk + i) * KP + 16 * nt + lm] = h;
-      pl[(4 * lk + i) * KP + 16 * nt + lm] = (_Float16)(p - (float)h);
-    }
-  // (a wave's LDS operations complete in order: its reads below see these stores)
-  att_f4 oacc[D / 16];
-#pragma unroll
-  for (int nt = 0; nt < D / 16; nt++) oacc[nt] = att_f4{0.0f, 0.0f, 0.0f, 0.0f};
-#pragma unroll
-  for (int ks = 0; ks < kChunkKeys / 32; ks++) {
-    const att_h8 ah = *(const att_h8*)(ph + lm * KP + 32 * ks + 8 * lk);
-    const att_h8 al = *(const att_h8*)(pl + lm * KP + 32 * ks + 8 * lk);
-#pragma unroll
-    for (int nt = 0; nt < D / 16; nt++) {
-      const att_h8 b = *(const att_h8*)(Vt + (16 * nt + lm) * KP + 32 * ks + 8 * lk);
-      oacc[nt] = att_mfma(ah, b, oacc[nt]);
-      oacc[nt] = att_mfma(al, b, oacc[nt]);
-    }
-  }
-  // the slot of (token, head): as attend_split_kernel
-#pragma unroll
-  for (int i = 0; i < 4; i++) {
-    if (!rowlive[i]) continue;
-    const int r = row0 + 4 * lk + i, t = t0 + r / GROUP, h = kvh * GROUP + r % GROUP;
-    const int64_t slot = ((int64_t)t * heads + h) * max_chunks + c;
-#pragma unroll
-    for (int nt = 0; nt < D / 16; nt++) part_acc[slot * D + 16 * nt + lm] = oacc[nt][i] * kPDrop;
-    if (lm == 0) {
-      part_ml[slot * 2 + 0] = mrow[i];
-      part_ml[slot * 2 + 1] = lrow[i];
-    }
-  }
-}
 
 // The same slice over a q8_0 cache (repack.mojo:181 CACHE_Q8): a position's
 // row is kv_width signed bytes, then kv_width/32 float16 factors, `row`
@@ -1034,7 +846,7 @@ __global__ __launch_bounds__(NT) void attend_wide_kernel(
 // attend_mfma_kernel: the same slice as attend_wide_kernel (one 64-key
 // slice x one key head x one token, f16 cache, GROUP <= 4 query heads of
 // head_dim D), with both products on the matrix cores
-// (v_mfma_f32_16x16x32_f16), as attend_chunk_kernel computes them for a
+// (v_mfma_f32_16x16x32_f16), as attend_flash.hip computes them for a
 // prefill chunk.  At 4 and 8 sequences the VALU dot loops of the wide
 // kernel bound its time; here a block of 256 threads does
 //   * S = K Q^T: wave w takes keys 16w..16w+15 as the A rows, read straight
@@ -1785,41 +1597,13 @@ int launch_attend(hipStream_t s, const float* q, int64_t q_stride, const uint16_
     return launch_merge(s, part_acc, part_ml, heads, head_dim, pos_dev, count_host, chunks, tokens, out, xq_out,
                         hx_out);
   }
-  // one sequence's chunk (its tokens share one cache): 16 tokens per block
-  // over one staged slice (f16 form; the q8 kernel takes one token a block)
+  // one sequence's chunk (its tokens share one cache): the flash kernel at head
+  // widths 64 and 128, else 16 tokens per block over one staged slice (f16
+  // form; the q8 kernel takes one token a block)
   const bool one_seq = kv_index ? index_stride == 0 : cache_stride == 0;
-  if (one_seq && pos_dev && tokens > kMaxTokens && form != MI_CACHE_Q8 && kk == kChunkKeys &&
-      (head_dim == 64 || head_dim == 128)) {
-    // a prefill chunk: the matrix-core slice kernel, then the same merge
-    dim3 cgrid(chunks, kv_heads, (tokens + 64 / group - 1) / (64 / group));
-    const size_t lds = attn_chunk_lds_bytes(head_dim);
-    // more than 64 KB of dynamic LDS has to be asked for, once per kernel and device
-#define MI_CHUNK(G, DD)                                                                                        \
-  {                                                                                                            \
-    static bool done[kMaxDevices];                                                                            \
-    if (int rc = allow_lds((const void*)attend_chunk_kernel<G, DD>, (int)attn_chunk_lds_bytes(DD), done,      \
-                           "attend_chunk LDS size"))                                                          \
-      return rc;                                                                                              \
-    hipLaunchKernelGGL((attend_chunk_kernel<G, DD>), cgrid, dim3(256), lds, s, q, q_stride,                    \
-                       (const __half*)k_cache, (const __half*)v_cache, heads, kv_heads, scale, pos_dev, chunks, \
-                       part_acc, part_ml, kv_index, tokens);                                                   \
-  }
-#define MI_CHUNK_D(G) \
-  if (head_dim == 64) MI_CHUNK(G, 64) else MI_CHUNK(G, 128)
-    switch (group) {
-      case 1: MI_CHUNK_D(1); break;
-      case 2: MI_CHUNK_D(2); break;
-      case 4: MI_CHUNK_D(4); break;
-      case 8: MI_CHUNK_D(8); break;
-      default: return fail(MI_ERR_SHAPE, "attend: %d query heads per key head is not 1, 2, 4 or 8", group);
-    }
-#undef MI_CHUNK_D
-#undef MI_CHUNK
-    int rc = hip_check(hipGetLastError(), "attend_chunk launch");
-    if (rc) return rc;
-    return launch_merge(s, part_acc, part_ml, heads, head_dim, pos_dev, count_host, chunks, tokens, out, xq_out,
-                        hx_out);
-  }
+  if (one_seq && pos_dev && out && !xq_out && flash_fits(heads, kv_heads, head_dim, tokens))
+    return launch_attend_flash(s, q, q_stride, k_cache, v_cache, heads, kv_heads, head_dim, scale, pos_dev, max_count,
+                               tokens, out, part_acc, part_ml, form, kv_index);
   const int tq = (one_seq && tokens > kMaxTokens && form != MI_CACHE_Q8) ? 16 : 1;
   dim3 grid(chunks, kv_heads, (tokens + tq - 1) / tq);
   const __half* kc = (const __half*)k_cache;

@@ -1,0 +1,93 @@
+"""A prompt chunk's attention (attend_flash.hip) at the sizes where it can go
+wrong: a chunk that starts at 0 and one that starts inside a 64-key slice, one
+slice (no split of the keys) and several, fewer tokens than a block's rows
+and more, every group size, both head widths, both cache forms, contiguous and
+paged, positions that are not held, a negative attention scale.
+
+The layer over the chunk is checked at its first tokens, its last and some
+between, against the oracle run on that token alone over the rows the device
+stored for the chunk's earlier tokens (the gate of tests/test_gpu_layer.py).
+"""
+
+import numpy as np
+import pytest
+import torch
+
+import oracle
+from molla_amd import synth
+from tests.test_gpu_layer import assert_layer_close, device_layer_from, layer_gate, make_layer_weights, spec_of
+
+pytestmark = pytest.mark.gpu
+
+CASES = [
+    # (width, hidden, heads, kv_heads, head_dim), first position, tokens
+    ((256, 256, 4, 4, 64), 0, 9),       # one slice: the finished row, no second launch
+    ((256, 256, 4, 4, 64), 55, 130),    # group 1: two blocks of rows, a slice's edge inside the chunk
+    ((256, 256, 2, 1, 128), 64, 64),    # group 2, whole slices
+    ((512, 256, 8, 2, 64), 190, 33),    # group 4, a block's rows one token past full
+    ((512, 256, 8, 1, 64), 1, 63),      # group 8
+    ((1024, 256, 8, 1, 128), 300, 17),  # group 8, one token past a block
+]
+
+
+@pytest.mark.parametrize("form", ["f16", "q8"])
+@pytest.mark.parametrize("dims,first,tokens", CASES)
+@pytest.mark.parametrize("paged", [False, True])
+def test_chunk_attention_edges(form, dims, first, tokens, paged):
+    from molla_amd import block, gpu
+    from tests.test_gpu_kernels import q8_decode, q8_rows
+    ctx = gpu.DeviceContext(0)
+    q8 = form == "q8"
+    f = gpu.CACHE_Q8 if q8 else gpu.CACHE_F16
+    spec = spec_of(*dims)
+    if first == 190:
+        spec["attn_scale"] = -spec["attn_scale"]
+    host = make_layer_weights(spec, 23)
+    host["attn_norm"] = (host["attn_norm"] * 0.05).astype(np.float32)  # scores of a model's size
+    # no MLP: behind random weights it magnifies a last bit of the attention
+    # (the oracle's own rounding of the token's key is 30 times the gate there)
+    kind, r, c, blob = host["down"]
+    host["down"] = (kind, r, c, np.zeros_like(blob))
+    bs, layer = device_layer_from(host, spec)
+    layer.desc.attn_scale = spec["attn_scale"]
+    kvw, count = bs.kv_width(), first + tokens
+    row = gpu.cache_row(f, kvw)
+    raw = [synth.normal(count * kvw, 90 + i).numpy().reshape(count, kvw) for i in (0, 1)]
+    rows = [q8_rows(r, kvw).reshape(count, row) if q8 else r.astype(np.float16).view(np.uint16) for r in raw]
+    x = synth.normal(tokens * bs.width, 92).numpy()
+    xd = torch.from_numpy(x.copy()).cuda()
+    posd = torch.arange(first, count, dtype=torch.int32, device="cuda")
+
+    def dev(a):
+        return torch.from_numpy(np.ascontiguousarray(a).view(np.int16)).view(torch.float16).cuda()
+
+    held = np.ones(count, bool)
+    if paged:
+        held[1:first:7] = False  # positions trimmed out of the window
+        order = np.random.default_rng(3).permutation(count + 5)[:count].astype(np.int32)
+        pools = [np.zeros((count + 5, row), np.uint16) for _ in rows]
+        for p, r in zip(pools, rows):
+            p[order] = r
+        kd, vd = (dev(p.reshape(-1)) for p in pools)
+        idx = torch.from_numpy(np.where(held, order, -1).astype(np.int32)).cuda()
+        block.device_layer_paged(ctx, layer, xd, kd, vd, idx, 0, posd, count, tokens, form=f)
+    else:
+        order = np.arange(count)
+        kd, vd = (dev(r.reshape(-1)) for r in rows)
+        block.device_layer(ctx, layer, xd, kd, vd, 0, posd, count, tokens, form=f)
+    ctx.synchronize()
+    got = [c.cpu().view(torch.int16).numpy().view(np.uint16).reshape(-1, row)[order] for c in (kd, vd)]
+    got = [q8_decode(g.reshape(-1), kvw, count) if q8 else g.view(np.float16).astype(np.float32) for g in got]
+    keep = []
+    L = oracle.make_layer(spec, host, keep)
+    for i in sorted({0, 1, 8, tokens // 2, tokens - 2, tokens - 1}):
+        p = first + i
+        kept = [j for j in range(p) if held[j]]
+        slot = len(kept)
+        kr, vr = (np.concatenate([g[kept], np.zeros((1, kvw), np.float32)]).astype(np.float32).reshape(-1) for g in got)
+        xr = x.reshape(tokens, -1)[i].copy()
+        # the oracle's own position is the slot count: give the float64 layer
+        # the kept rows, the rope the true position
+        bound = layer_gate(spec, host, xr, kr, vr, slot)
+        oracle.layer_step(L, xr, kr, vr, slot, p, f16_store=not q8, q8_store=q8, threads=8)
+        assert_layer_close(xd.cpu().numpy().reshape(tokens, -1)[i], xr, bound, f"token {i}:")
