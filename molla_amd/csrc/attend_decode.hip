@@ -1,0 +1,444 @@
+// attend_decode.hip -- decode attention on the matrix cores
+// (v_mfma_f32_16x16x32_f16), gfx950: attention.mojo:144 attend for one query
+// token per sequence, over an f16 or a q8_0 cache (gpu_ops.mojo:678
+// attend_kernel's `form`), GQA with up to 8 query heads a key head, head_dim
+// 64 or 128; the split and the fold of gpu_ops.mojo:929 / 1104.
+//
+// A block takes a share of one (key head, token)'s keys; each of its four
+// waves walks every fourth 32-key run of the share by itself, with a running
+// maximum and sum in registers and its own LDS rows for the values (no block
+// barrier until the waves' results are folded at the end), and sends for the
+// next run's keys and values as soon as it has used this one's.  The number of
+// shares fills the chip and stays at 64, so a long context costs a few partial
+// results a head and not one a 64-key slice.  us for the shares + the fold (the
+// 64-key slices' kernel + merge before), 32 heads of 128 over 8 key heads:
+// 32768 keys f16, cold, 34.6 + 4.6 (34.4 + 21.4: 134 MB at 3.9 TB/s, near the
+// read rate); 4097 keys 7.7 + 3.6 (6.7 + 6.0: latency, one run a wave); 8
+// sequences of 4700 keys, paged q8_0, 34.7 + 4.7 (51.1 + 7.3: the loads' latency
+// at two waves a SIMD, 2.4 TB/s).
+//
+//   S^T = K Q^T, keys as rows (read straight from the cache) and queries as
+//   columns: a lane's 8 scores belong to its own query, the softmax takes two
+//   exchanges between lanes, and the weights are in place as the B operand of
+//   O^T = V^T P^T.  Queries enter as three halves (every bit of the f32), P as
+//   two after a lift by 2^14; values lie by rows in LDS and are read
+//   transposed (ds_read_b64_tr_b16).  Slot i of lane group g takes key
+//   4 g + i % 4 + 16 (i / 4), the order in which S^T leaves them.
+//
+// q8_0: quants enter as exact halves; a key block's factor multiplies its part
+// of the score, a value block's the weights, held relative to the largest
+// factor so far of that block of 32 dims (2^-X) so that no half is subnormal.
+//
+// MFMA fragments (16x16x32): lane l holds row / column l % 16 and values
+// 8 (l / 16) .. +8 of the 32; result element i of lane l is row 4 (l / 16) +
+// i, column l % 16.
+#include <math.h>
+
+#include <algorithm>
+
+#include "mi_internal.h"
+
+namespace mi {
+namespace {
+
+typedef _Float16 dh2 __attribute__((ext_vector_type(2)));
+typedef _Float16 dh8 __attribute__((ext_vector_type(8)));
+typedef short ds4 __attribute__((ext_vector_type(4)));
+typedef short ds8 __attribute__((ext_vector_type(8)));
+typedef float df4 __attribute__((ext_vector_type(4)));
+typedef uint32_t du4 __attribute__((ext_vector_type(4)));
+typedef uint32_t du2 __attribute__((ext_vector_type(2)));
+
+constexpr int kRun = 32;            // keys a wave takes at a time
+constexpr int kWaves = 4;           // waves a block
+constexpr int kStep = kRun * kWaves;  // keys a block takes at a time
+constexpr int kMaxShares = 64;
+constexpr float kLift = 14.0f;      // P in [0, 2^14]: see attend_flash.hip
+constexpr float kLog2e = 1.44269504088896340736f;
+
+__device__ __forceinline__ df4 mfma16(dh8 a, dh8 b, df4 c) {
+  return __builtin_amdgcn_mfma_f32_16x16x32_f16(a, b, c, 0, 0, 0);
+}
+
+// 16-byte piece pc of LDS row r lies at slot pc ^ swz(r): a transposed read
+// takes 4 rows x 32 bytes per 16 lanes, on distinct banks.
+template <int D>
+__device__ __forceinline__ int swz(int r) {
+  return (D == 128 ? 4 * (r & 3) : 4 * ((r >> 1) & 1)) | ((r >> 2) & 3);
+}
+
+// over the four lanes that share a column
+template <class Op>
+__device__ __forceinline__ float across(float v, Op op) {
+  auto p = __builtin_amdgcn_permlane16_swap(__float_as_uint(v), __float_as_uint(v), false, false);
+  v = op(__uint_as_float(p[0]), __uint_as_float(p[1]));
+  p = __builtin_amdgcn_permlane32_swap(__float_as_uint(v), __float_as_uint(v), false, false);
+  return op(__uint_as_float(p[0]), __uint_as_float(p[1]));
+}
+
+__device__ __forceinline__ dh2 as_dh2(uint32_t u) { return __builtin_bit_cast(dh2, u); }
+
+// eight signed bytes as halves: 0x64 above byte + 128 is 1152 + byte
+__device__ __forceinline__ dh8 int8_halves(uint32_t x, uint32_t y) {
+  const dh2 off = {(_Float16)-1152.0f, (_Float16)-1152.0f};
+  x ^= 0x80808080u;
+  y ^= 0x80808080u;
+  const du4 m = {__builtin_amdgcn_perm(0x64646464u, x, 0x04010400u), __builtin_amdgcn_perm(0x64646464u, x, 0x04030402u),
+                 __builtin_amdgcn_perm(0x64646464u, y, 0x04010400u), __builtin_amdgcn_perm(0x64646464u, y, 0x04030402u)};
+  du4 r;
+#pragma unroll
+  for (int i = 0; i < 4; i++) r[i] = __builtin_bit_cast(uint32_t, as_dh2(m[i]) + off);
+  return __builtin_bit_cast(dh8, r);
+}
+
+// The grid is (shares, kv_heads, tokens); share s takes the s-th part of the
+// 128-key steps that the token's own count has (a device value: the host
+// knows only the context) and writes each head's unnormalised sum with
+// (maximum, sum) in base 2 to slot (token, head, share); (0, 0) for no keys.
+template <int D, bool Q8, bool PAGED>
+__global__ __launch_bounds__(64 * kWaves, 2) void attend_decode_kernel(
+    const float* __restrict__ q, int64_t q_stride, const __half* __restrict__ kc, const __half* __restrict__ vc,
+    int64_t cache_stride, int row_halves, int heads, int kv_heads, int group, float scale,
+    const int32_t* __restrict__ pos, int count_host, const int32_t* __restrict__ kv_index, int64_t index_stride,
+    float* __restrict__ part_acc, float* __restrict__ part_ml) {
+  constexpr int KS = D / 32, NT = D / 16, PIECES = D / 8;
+  constexpr int kFac = Q8 ? 2 * KS * kRun : 1;             // floats: factors of a run's keys and values
+  constexpr int kWaveBytes = kRun * D * 2;                 // a run's values as halves
+  __shared__ __align__(16) uint8_t vs[kWaves][kWaveBytes];  // afterwards the waves' sums
+  __shared__ __align__(16) float fac[kWaves][kFac];
+  __shared__ float wml[kWaves][2][16];
+  static_assert(8 * D * 4 <= kWaveBytes, "a wave's sums of 8 heads in place of its values");
+  const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+  const int lm = lane & 15, lk = lane >> 4;
+  const int share = blockIdx.x, shares = gridDim.x, kvh = blockIdx.y, t = blockIdx.z;
+  const int count = pos ? pos[t] + 1 : count_host;
+  const int steps = (count + kStep - 1) / kStep, per = (steps + shares - 1) / shares;
+  const int s0 = share * per, s1 = min(s0 + per, steps);
+  const int64_t slot0 = ((int64_t)t * heads + (int64_t)kvh * group) * shares + share;
+  if (s0 >= s1) {
+    if (tid < group) *(float2*)(part_ml + (slot0 + (int64_t)tid * shares) * 2) = make_float2(0.0f, 0.0f);
+    return;
+  }
+  if (PAGED) kv_index += t * index_stride;
+  const int64_t seq = PAGED ? 0 : (int64_t)t * cache_stride;
+  const int kvw = kv_heads * D;
+  // The cells of a run's keys, key lane % 32 a lane (keys past the end repeat
+  // the last one, masked below): read a run ahead of its keys and values, which
+  // take theirs from the lane that has it
+  auto cells_of = [&](int key) __attribute__((always_inline)) {
+    const int j = min(key + (lane & 31), count - 1);
+    return PAGED ? kv_index[j] : j;
+  };
+  auto row_of = [&](int key, int cells, int r) __attribute__((always_inline)) {
+    const int cell = PAGED ? max(__shfl(cells, r), 0) : min(key + r, count - 1);
+    return seq + (int64_t)cell * row_halves;
+  };
+
+  // the queries, first in line: column lm (past the group, the last one)
+  const float* qr = q + (int64_t)t * q_stride + ((int64_t)kvh * group + min(lm, group - 1)) * D + 8 * lk;
+  df4 qraw[KS][2];
+#pragma unroll
+  for (int ks = 0; ks < KS; ks++) {
+    qraw[ks][0] = *(const df4*)(qr + 32 * ks);
+    qraw[ks][1] = *(const df4*)(qr + 32 * ks + 4);
+  }
+
+  // a run's keys (lane: key lm of each 16-key tile, its values 32 ks + 8 lk ..
+  // +8), values (16-byte pieces of its rows) and q8_0 factors (lane: key
+  // lane % 32, keys' below lane 32 and values' above)
+  typedef typename std::conditional<Q8, du2, du4>::type KWord;
+  constexpr int VW = Q8 ? kRun * D / 16 / 64 : kRun * PIECES / 64;
+  KWord kw[2][KS];
+  du4 vw[VW];
+  du2 fw = {0, 0};
+  auto load_k = [&](int key0, int cells) __attribute__((always_inline)) {
+#pragma unroll
+    for (int a = 0; a < 2; a++) {
+      const __half* r = kc + row_of(key0, cells, 16 * a + lm);
+#pragma unroll
+      for (int ks = 0; ks < KS; ks++)
+        kw[a][ks] = Q8 ? *(const KWord*)((const int8_t*)r + kvh * D + 32 * ks + 8 * lk)
+                       : *(const KWord*)(r + kvh * D + 32 * ks + 8 * lk);
+    }
+  };
+  auto load_v = [&](int key0, int cells) __attribute__((always_inline)) {
+    if constexpr (Q8) {
+      const __half* c = (lane < 32 ? kc : vc) + row_of(key0, cells, lane & 31) + (kvw >> 1) + ((kvh * D) >> 5);
+      if constexpr (KS == 4) fw = *(const du2*)c;
+      else fw.x = *(const uint32_t*)c;
+    }
+#pragma unroll
+    for (int j = 0; j < VW; j++) {
+      const int i = lane + 64 * j;
+      if constexpr (Q8) vw[j] = *(const du4*)((const int8_t*)(vc + row_of(key0, cells, i / (D / 16))) + kvh * D + 16 * (i % (D / 16)));
+      else vw[j] = *(const du4*)(vc + row_of(key0, cells, i / PIECES) + kvh * D + 8 * (i % PIECES));
+    }
+  };
+  int key0 = s0 * kStep + kRun * wave;
+  int cells = cells_of(key0);
+  load_k(key0, cells);
+  load_v(key0, cells);
+  int cells_next = cells_of(key0 + kStep);
+  __builtin_amdgcn_sched_barrier(0);
+
+  // the queries as B fragments: column lm (zero past the group)
+  const float c2 = fabsf(scale) * kLog2e;
+  dh8 qf[3][KS];
+  {
+    const float sgn = scale < 0.0f ? -1.0f : 1.0f;
+#pragma unroll
+    for (int ks = 0; ks < KS; ks++) {
+#pragma unroll
+      for (int u = 0; u < 8; u++) {
+        const float f = lm < group ? sgn * qraw[ks][u >> 2][u & 3] : 0.0f;
+        const _Float16 h1 = (_Float16)f;
+        const float r1 = f - (float)h1;  // exact
+        const _Float16 h2 = (_Float16)r1;
+        qf[0][ks][u] = h1;
+        qf[1][ks][u] = h2;
+        qf[2][ks][u] = (_Float16)(r1 - (float)h2);
+      }
+    }
+  }
+
+  typedef __attribute__((address_space(3))) char* lds_ptr;
+  const lds_ptr vl = (lds_ptr)&vs[wave][0];
+  float* fl = fac[wave];
+  // transposed reads: rows 4 lk + i16 / 4 (+ 16), dims 16 dt + 4 (i16 % 4): the
+  // slot is an exclusive or with bits a row's start leaves free
+  uint32_t vat[2];
+#pragma unroll
+  for (int v = 0; v < 2; v++) {
+    const int row = 4 * lk + (lm >> 2) + 16 * v;
+    vat[v] = 2 * row * D + 16 * (((lm & 3) >> 1) ^ swz<D>(row)) + 8 * (lm & 1);
+  }
+  df4 o[NT];
+#pragma unroll
+  for (int dt = 0; dt < NT; dt++) o[dt] = df4{0.0f, 0.0f, 0.0f, 0.0f};
+  int xo[Q8 ? KS : 1];  // q8_0: the X that each 32-dim block of o is held at
+#pragma unroll
+  for (int b = 0; b < (Q8 ? KS : 1); b++) xo[b] = -100;
+  float mc = -1e30f, l = 0.0f;
+
+  for (int sl = s0; sl < s1; sl++, key0 += kStep) {
+    if (key0 >= count) break;  // (uniform over the wave: no keys left for it)
+    df4 s[2];
+    if constexpr (Q8) {
+      // factors to LDS by (key | value, block, key), read back four keys a lane
+#pragma unroll
+      for (int b = 0; b < KS; b++)
+        fl[(lane >> 5) * KS * kRun + b * kRun + (lane & 31)] = half_bits_to_float(b < 2 ? fw.x >> (16 * b) : fw.y >> (16 * (b - 2)));
+      asm volatile("" ::: "memory");
+#pragma unroll
+      for (int a = 0; a < 2; a++) {
+        s[a] = df4{0.0f, 0.0f, 0.0f, 0.0f};
+#pragma unroll
+        for (int ks = 0; ks < KS; ks++) {
+          const dh8 k8 = int8_halves(kw[a][ks].x, kw[a][ks].y);
+          df4 c = {0.0f, 0.0f, 0.0f, 0.0f};
+#pragma unroll
+          for (int h = 0; h < 3; h++) c = mfma16(k8, qf[h][ks], c);
+          const df4 f = *(const df4*)(fl + ks * kRun + 16 * a + 4 * lk);
+#pragma unroll
+          for (int i = 0; i < 4; i++) s[a][i] = fmaf(f[i], c[i], s[a][i]);
+        }
+      }
+    } else {
+#pragma unroll
+      for (int a = 0; a < 2; a++) {
+        s[a] = df4{0.0f, 0.0f, 0.0f, 0.0f};
+#pragma unroll
+        for (int ks = 0; ks < KS; ks++)
+#pragma unroll
+          for (int h = 0; h < 3; h++) s[a] = mfma16(__builtin_bit_cast(dh8, kw[a][ks]), qf[h][ks], s[a]);
+      }
+    }
+    uint32_t held = 0xffffffffu;
+    if constexpr (PAGED) held = (uint32_t)__ballot(cells >= 0);
+    const int nk = min(kRun, count - key0);
+    if (nk < kRun) held &= (1u << nk) - 1u;
+    const bool more = key0 + kStep < count && sl + 1 < s1;  // uniform
+    if (more) load_k(key0 + kStep, cells_next);
+
+    // running maximum and weights of this lane's keys 16 a + 4 lk + i
+    const uint32_t mine = held >> (4 * lk);
+    float m = -INFINITY;
+#pragma unroll
+    for (int a = 0; a < 2; a++)
+#pragma unroll
+      for (int i = 0; i < 4; i++) {
+        s[a][i] = (mine >> (16 * a + i)) & 1 ? s[a][i] : -INFINITY;
+        m = fmaxf(m, s[a][i]);
+      }
+    m = across(m, lanes::Max{});
+    const float mn = fmaxf(mc, m == -INFINITY ? -1e30f : m * c2);
+    if (__any(mn != mc)) {
+      const float f = __builtin_amdgcn_exp2f(mc - mn);
+      l *= f;
+#pragma unroll
+      for (int dt = 0; dt < NT; dt++) o[dt] *= f;
+      mc = mn;
+    }
+    float p[8];
+#pragma unroll
+    for (int a = 0; a < 2; a++)
+#pragma unroll
+      for (int i = 0; i < 4; i++) {
+        const float e = __builtin_amdgcn_exp2f(fmaf(s[a][i], c2, kLift - mc));
+        p[4 * a + i] = (mine >> (16 * a + i)) & 1 ? e : 0.0f;
+        l += p[4 * a + i];
+      }
+
+    // the values to this wave's LDS rows
+#pragma unroll
+    for (int j = 0; j < VW; j++) {
+      const int i = lane + 64 * j;
+      if constexpr (Q8) {
+        const int row = i / (D / 16), pc = 2 * (i % (D / 16));
+        *(__attribute__((address_space(3))) dh8*)(vl + 2 * row * D + 16 * (pc ^ swz<D>(row))) = int8_halves(vw[j].x, vw[j].y);
+        *(__attribute__((address_space(3))) dh8*)(vl + 2 * row * D + 16 * ((pc + 1) ^ swz<D>(row))) = int8_halves(vw[j].z, vw[j].w);
+      } else {
+        const int row = i / PIECES, pc = i % PIECES;
+        *(__attribute__((address_space(3))) du4*)(vl + 2 * row * D + 16 * (pc ^ swz<D>(row))) = vw[j];
+      }
+    }
+    df4 fv[Q8 ? KS : 1][2];
+    if constexpr (Q8) {
+#pragma unroll
+      for (int b = 0; b < KS; b++)
+#pragma unroll
+        for (int a = 0; a < 2; a++) fv[b][a] = *(const df4*)(fl + KS * kRun + b * kRun + 16 * a + 4 * lk);
+    }
+    asm volatile("" ::: "memory");  // (a wave's LDS operations complete in order)
+    if (more) load_v(key0 + kStep, cells_next);
+    cells = cells_next;
+    cells_next = cells_of(key0 + 2 * kStep);
+
+    dh8 ph, pl;
+    if constexpr (!Q8) {
+#pragma unroll
+      for (int i = 0; i < 8; i++) {
+        ph[i] = (_Float16)p[i];
+        pl[i] = (_Float16)(p[i] - (float)ph[i]);
+      }
+    }
+#pragma unroll
+    for (int dt = 0; dt < NT; dt++) {
+      if constexpr (Q8) {
+        if (dt % 2 == 0) {
+          const int b = dt / 2;
+          float fm = 0.0f;
+#pragma unroll
+          for (int i = 0; i < 8; i++) fm = fmaxf(fm, fabsf(fv[b][i >> 2][i & 3]));
+          fm = across(fm, lanes::Max{});
+          const int x = __builtin_amdgcn_readfirstlane(fm > 0.0f ? max(xo[b], __builtin_amdgcn_frexp_expf(fm)) : xo[b]);
+          if (x != xo[b]) {
+            const float f = ldexpf(1.0f, xo[b] - x);
+            o[dt] *= f;
+            o[dt + 1] *= f;
+            xo[b] = x;
+          }
+          const float unit = ldexpf(1.0f, -x);
+#pragma unroll
+          for (int i = 0; i < 8; i++) {
+            // rounded once: contracted into the two conversions, the halves
+            // came from two roundings of the product, a last bit of hi apart
+            float w = p[i] * (fv[b][i >> 2][i & 3] * unit);
+            asm("" : "+v"(w));
+            ph[i] = (_Float16)w;
+            pl[i] = (_Float16)(w - (float)ph[i]);
+          }
+        }
+      }
+      ds8 a;
+#pragma unroll
+      for (int v = 0; v < 2; v++) {
+        const ds4 x = __builtin_amdgcn_ds_read_tr16_b64_v4i16(
+            (__attribute__((address_space(3))) ds4*)(vl + (vat[v] ^ (32 * dt))));
+#pragma unroll
+        for (int e = 0; e < 4; e++) a[4 * v + e] = x[e];
+      }
+      o[dt] = mfma16(__builtin_bit_cast(dh8, a), ph, o[dt]);
+      o[dt] = mfma16(__builtin_bit_cast(dh8, a), pl, o[dt]);
+    }
+    asm volatile("" ::: "memory");  // the reads above stay ahead of the next run's stores
+  }
+
+  // fold the waves: their sums (in place of the values) and (maximum, sum)
+  l = across(l, lanes::Add{});
+  float* wo = (float*)&vs[0][0];  // [wave][group][D]
+  __syncthreads();
+  if (lm < group) {
+#pragma unroll
+    for (int dt = 0; dt < NT; dt++) {
+      if constexpr (Q8) o[dt] *= ldexpf(1.0f, xo[dt / 2]);
+      *(df4*)(wo + (wave * group + lm) * D + 16 * dt + 4 * lk) = o[dt];
+    }
+    if (lk == 0) {
+      wml[wave][0][lm] = mc;
+      wml[wave][1][lm] = l;
+    }
+  }
+  __syncthreads();
+  for (int i = tid; i < group * D; i += 64 * kWaves) {
+    const int g = i / D, d = i - g * D;
+    float m = wml[0][0][g];
+#pragma unroll
+    for (int w = 1; w < kWaves; w++) m = fmaxf(m, wml[w][0][g]);
+    float v = 0.0f, sum = 0.0f;
+#pragma unroll
+    for (int w = 0; w < kWaves; w++) {
+      const float f = __builtin_amdgcn_exp2f(wml[w][0][g] - m);
+      v = fmaf(wo[(w * group + g) * D + d], f, v);
+      sum = fmaf(wml[w][1][g], f, sum);
+    }
+    const int64_t slot = slot0 + (int64_t)g * shares;
+    part_acc[slot * D + d] = v;
+    if (d == 0) *(float2*)(part_ml + slot * 2) = make_float2(m, sum);
+  }
+}
+
+}  // namespace
+
+bool decode_attend_fits(int32_t group, int32_t head_dim) {
+  return (group == 1 || group == 2 || group == 4 || group == 8) && (head_dim == 64 || head_dim == 128);
+}
+
+// Shares of the keys: about four blocks a compute unit, at most one a 128-key
+// step of the context and 64 (the fold takes them in one round).
+int decode_attend_shares(int32_t kv_heads, int32_t tokens, int32_t max_count) {
+  const int steps = (max_count + kStep - 1) / kStep;
+  const int want = (4 * cu_count() + kv_heads * tokens - 1) / (kv_heads * tokens);
+  return std::max(1, std::min({want, steps, kMaxShares}));
+}
+
+int launch_attend_decode(hipStream_t s, const float* q, int64_t q_stride, const uint16_t* k_cache,
+                         const uint16_t* v_cache, int64_t cache_stride, int32_t heads, int32_t kv_heads,
+                         int32_t head_dim, float scale, const int32_t* pos, int32_t count_host, int32_t shares,
+                         int32_t tokens, float* part_acc, float* part_ml, int32_t form, const int32_t* kv_index,
+                         int64_t index_stride) {
+  const int row = cache_row(form, kv_heads * head_dim);
+  const dim3 grid(shares, kv_heads, tokens);
+#define MI_DEC(DD, Q, P)                                                                                         \
+  hipLaunchKernelGGL((attend_decode_kernel<DD, Q, P>), grid, dim3(64 * kWaves), 0, s, q, q_stride,                 \
+                     (const __half*)k_cache, (const __half*)v_cache, cache_stride, row, heads, kv_heads,           \
+                     heads / kv_heads, scale, pos, count_host, kv_index, index_stride, part_acc, part_ml)
+#define MI_DEC_F(DD)                         \
+  if (form == MI_CACHE_Q8) {                 \
+    if (kv_index) MI_DEC(DD, true, true);    \
+    else MI_DEC(DD, true, false);            \
+  } else {                                   \
+    if (kv_index) MI_DEC(DD, false, true);   \
+    else MI_DEC(DD, false, false);           \
+  }
+  if (head_dim == 64) {
+    MI_DEC_F(64)
+  } else {
+    MI_DEC_F(128)
+  }
+#undef MI_DEC_F
+#undef MI_DEC
+  return hip_check(hipGetLastError(), "attend_decode launch");
+}
+
+}  // namespace mi

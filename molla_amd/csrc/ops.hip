@@ -479,21 +479,6 @@ __global__ __launch_bounds__(kAttnThreads) void attend_split_kernel(
   }
 }
 
-// MFMA fragments (16x16x32): lane l holds row/column l % 16 and values
-// 8 (l / 16) .. +8 of the 32; the result element i of lane l is row
-// 4 (l / 16) + i, column l % 16.
-typedef _Float16 att_h8 __attribute__((ext_vector_type(8)));
-typedef float att_f4 __attribute__((ext_vector_type(4)));
-
-__device__ __forceinline__ att_f4 att_mfma(att_h8 a, att_h8 b, att_f4 c) {
-  return __builtin_amdgcn_mfma_f32_16x16x32_f16(a, b, c, 0, 0, 0);
-}
-
-// The matrix-core slice splits P (at most 1) into two halves after lifting
-// it by 2^14, and scale the sums back: exact powers of two, which keep the
-// low halves of weights down to ~1e-8 out of the f16 subnormals.
-constexpr float kPLift = 16384.0f, kPDrop = 1.0f / 16384.0f;
-
 // The same slice over a q8_0 cache (repack.mojo:181 CACHE_Q8): a position's
 // row is kv_width signed bytes, then kv_width/32 float16 factors, `row`
 // halves in all.  Quants and factors are staged in LDS as they are (half the
@@ -650,7 +635,10 @@ __global__ __launch_bounds__(256) void store_kv_q8_kernel(const float* __restric
 // further rounds past it): each up-front load is an instruction of every
 // thread, and 64 of them where 36 slices are live made a decode step
 // 12-32 us slower (batch 1 to 8) than 40 or 48.
-template <int B>
+// FOLD: the slices are attend_decode.hip's shares, max_chunks of them whatever
+// the position, their maxima in base 2 and a sum of 0 where no key fell in
+// (whose values were never written).
+template <int B, bool FOLD>
 __global__ void attend_merge_kernel(const float* __restrict__ part_acc, const float* __restrict__ part_ml,
                                     int heads, int head_dim, const int32_t* __restrict__ pos_dev,
                                     int count_host, int max_chunks, float* __restrict__ out,
@@ -667,12 +655,12 @@ __global__ void attend_merge_kernel(const float* __restrict__ part_acc, const fl
   float2 ml = pml[min(lane, max_chunks - 1)];
   const int count = pos_dev ? pos_dev[t] + 1 : count_host;  // a position p attends over p + 1 slots
   const int kk = attn_slice(head_dim);
-  const int chunks = min((count + kk - 1) / kk, max_chunks);
+  const int chunks = FOLD ? max_chunks : min((count + kk - 1) / kk, max_chunks);
   // the largest slice max over every round
-  float M = lane < chunks ? ml.x : -INFINITY;
+  float M = lane < chunks && (!FOLD || ml.y != 0.0f) ? ml.x : -INFINITY;
   for (int c0 = B; c0 < chunks; c0 += B) {
     const int c = c0 + lane;
-    if (c < chunks) M = fmaxf(M, pml[c].x);
+    if (c < chunks && (!FOLD || pml[c].y != 0.0f)) M = fmaxf(M, pml[c].x);
   }
   M = lanes::reduce<64>(M, lanes::Max{});
   float o = 0.0f, L = 0.0f;
@@ -683,11 +671,13 @@ __global__ void attend_merge_kernel(const float* __restrict__ part_acc, const fl
       ml = pml[min(c0 + lane, chunks - 1)];
     }
     const int n = min(chunks - c0, B);
-    const float w = lane < n ? expf(ml.x - M) : 0.0f;
+    const float e = FOLD ? __builtin_amdgcn_exp2f(ml.x - M) : expf(ml.x - M);
+    const float w = lane < n && (!FOLD || ml.y != 0.0f) ? e : 0.0f;
     L += lane < n ? ml.y * w : 0.0f;
 #pragma unroll
     for (int k = 0; k < B; k++) {
-      if (k < n) o = fmaf(a[k], __int_as_float(__builtin_amdgcn_readlane(__float_as_int(w), k)), o);
+      const float wk = __int_as_float(__builtin_amdgcn_readlane(__float_as_int(w), k));
+      if (FOLD ? wk != 0.0f : k < n) o = fmaf(a[k], wk, o);
     }
   }
   L = lanes::reduce<64>(L, lanes::Add{});
@@ -698,494 +688,6 @@ __global__ void attend_merge_kernel(const float* __restrict__ part_acc, const fl
     quantize_group32(o, threadIdx.x & 31, (h * head_dim + d) >> 5, width >> 5,
                      xq + (int64_t)t * xq_token_bytes(width), live,
                      hx ? hx + (int64_t)t * xq_token_bytes(width) : nullptr);
-}
-
-// ---- decode attention slices ------------------------------------------------
-// attend_wide_kernel: the slice half of attention.mojo:144 attend
-// (gpu_ops.mojo:929 attend_split_kernel) for one query token per sequence
-// over an f16 cache, head_dim 64 or 128.  A block takes one (64-key slice,
-// key head, token) as attend_split_kernel does, with NT = 1024 threads (one
-// token; 512 for a batch, so that two blocks share a CU) instead of 256, so
-// every stage is spread over NT / 64 waves:
-//   * the slice's keys and values go to LDS with one load per thread;
-//   * each (query head, key) score is SPL threads of DPT dimensions each,
-//     added by shuffles;
-//   * the slice softmax is one wave per query head (lane = key);
-//   * each weighted value pair (query head, 2 dims) is KQ threads over
-//     interleaved keys, added by shuffles.
-// It writes each slice's (max, sum) and unnormalised values exactly where
-// attend_split_kernel does, and attend_merge_kernel folds them.
-constexpr int kWideKeys = 64;
-
-template <int GROUP, int D, int NT>
-struct WideShape {
-  static constexpr int KS = D + 8;   // K rows in halves (16-byte pad)
-  static constexpr int VS = D + 32;  // V rows: 16 dwords of pad, so the KQ lanes
-                                     // reading one dim pair hit distinct banks
-  static constexpr int SPL0 = NT / (GROUP * kWideKeys);
-  static constexpr int SPL = SPL0 < (D / 8) ? SPL0 : (D / 8);  // threads per score
-  static constexpr int DPT = D / SPL;                           // dims per score thread
-  static constexpr int KQ = 2 * NT / (GROUP * D);               // threads per output pair
-};
-
-template <int GROUP, int D, int NT>
-__global__ __launch_bounds__(NT) void attend_wide_kernel(
-    const float* __restrict__ q, int64_t q_stride, const __half* __restrict__ kc, const __half* __restrict__ vc,
-    int64_t cache_stride, int heads, int kv_heads, float scale, const int32_t* __restrict__ pos_dev,
-    int count_host, int max_chunks, float* __restrict__ part_acc, float* __restrict__ part_ml,
-    const int32_t* __restrict__ kv_index, int64_t index_stride) {
-  using S = WideShape<GROUP, D, NT>;
-  constexpr int KK = kWideKeys, PIECES = D / 8, TOTAL = KK * PIECES, PAIRS = D / 2;
-  constexpr int PER = (TOTAL + NT - 1) / NT;  // 16-byte pieces of K (and of V) per thread
-  static_assert(GROUP * D / 4 <= NT && S::SPL >= 1 && S::KQ >= 1 && S::KQ <= 64, "shape");
-  __shared__ __align__(16) __half Ks[KK * S::KS];
-  __shared__ __align__(16) __half Vs[KK * S::VS];
-  __shared__ __align__(16) float Qs[GROUP * D];
-  __shared__ float Ss[GROUP * KK];
-  const int c = blockIdx.x, kvh = blockIdx.y, t = blockIdx.z;
-  const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
-  const int count = pos_dev ? pos_dev[t] + 1 : count_host;  // a position p attends over p + 1 slots
-  const int start = c * KK;
-  if (start >= count) return;
-  const int nk = min(KK, count - start);
-  const int kvw = kv_heads * D;
-
-  // stage: the group's queries, one 16-byte piece of a key and of a value
-  // per thread (keys past the end repeat the last live one; masked below)
-  const float* qg = q + (int64_t)t * q_stride + (int64_t)kvh * GROUP * D;
-  const bool has_q = tid < GROUP * D / 4;
-  const float4 qv = ((const float4*)qg)[has_q ? tid : 0];
-  const int64_t seq = kv_index ? 0 : (int64_t)t * cache_stride;
-  uint4 kraw[PER], vraw[PER];
-#pragma unroll
-  for (int j = 0; j < PER; j++) {
-    const int i = min(tid + j * NT, TOTAL - 1);
-    const int skey = i / PIECES, pc = i % PIECES;
-    const int cell = max(kv_cell(kv_index, index_stride, t, start + min(skey, nk - 1)), 0);
-    const int64_t off = seq + (int64_t)cell * kvw + (int64_t)kvh * D + pc * 8;
-    kraw[j] = *(const uint4*)(kc + off);
-    vraw[j] = *(const uint4*)(vc + off);
-  }
-  if (has_q) ((float4*)Qs)[tid] = qv;
-#pragma unroll
-  for (int j = 0; j < PER; j++) {
-    const int i = tid + j * NT;
-    const int skey = i / PIECES, pc = i % PIECES;
-    if (i < TOTAL) {
-      *(uint4*)(Ks + skey * S::KS + pc * 8) = kraw[j];
-      *(uint4*)(Vs + skey * S::VS + pc * 8) = vraw[j];
-    }
-  }
-  __syncthreads();
-
-  // scores: thread = (query head g, key, part of DPT dims)
-  {
-    const int dot = tid / S::SPL, part = tid % S::SPL;
-    const int g = dot / KK, key = dot % KK;
-    float sdot = 0.0f;
-    if (dot < GROUP * KK) {
-      const __half* kr = Ks + key * S::KS + part * S::DPT;
-      const float* qq = Qs + g * D + part * S::DPT;
-#pragma unroll
-      for (int d = 0; d < S::DPT; d += 8) {
-        const uint4 raw = *(const uint4*)(kr + d);
-        const __half2* h2 = (const __half2*)&raw;
-        const float4 qa = *(const float4*)(qq + d), qb = *(const float4*)(qq + d + 4);
-        const float2 k0 = __half22float2(h2[0]), k1 = __half22float2(h2[1]);
-        const float2 k2 = __half22float2(h2[2]), k3 = __half22float2(h2[3]);
-        sdot = fmaf(qa.x, k0.x, sdot);
-        sdot = fmaf(qa.y, k0.y, sdot);
-        sdot = fmaf(qa.z, k1.x, sdot);
-        sdot = fmaf(qa.w, k1.y, sdot);
-        sdot = fmaf(qb.x, k2.x, sdot);
-        sdot = fmaf(qb.y, k2.y, sdot);
-        sdot = fmaf(qb.z, k3.x, sdot);
-        sdot = fmaf(qb.w, k3.y, sdot);
-      }
-    }
-    sdot = lanes::reduce<S::SPL>(sdot, lanes::Add{});
-    if (part == 0 && dot < GROUP * KK) {
-      const bool live = key < nk && (!kv_index || kv_cell(kv_index, index_stride, t, start + key) >= 0);
-      Ss[g * KK + key] = live ? sdot * scale : -INFINITY;
-    }
-  }
-  __syncthreads();
-  const int64_t slot0 = ((int64_t)t * heads + (int64_t)kvh * GROUP) * max_chunks;
-  // slice softmax: wave g takes query head g, lane = key
-  if (wave < GROUP) {
-    const float sc = Ss[wave * KK + lane];
-    float m = sc;
-    m = lanes::reduce<64>(m, lanes::Max{});
-    const float pr = sc == -INFINITY ? 0.0f : expf(sc - m);
-    float l = pr;
-    l = lanes::reduce<64>(l, lanes::Add{});
-    Ss[wave * KK + lane] = pr;
-    if (lane == 0) *(float2*)(part_ml + (slot0 + (int64_t)wave * max_chunks + c) * 2) = make_float2(m, l);
-  }
-  __syncthreads();
-  // unnormalised weighted values: thread = (query head, dim pair, key residue kq)
-  const int kq = tid % S::KQ, oe = tid / S::KQ;
-  const int g = oe / PAIRS, e = oe % PAIRS;
-  float a0 = 0.0f, a1 = 0.0f;
-  if (oe < GROUP * PAIRS) {
-    const float* pg = Ss + g * KK;
-#pragma unroll 4
-    for (int k = kq; k < KK; k += S::KQ) {
-      const float p = pg[k];
-      const float2 v = __half22float2(*(const __half2*)(Vs + k * S::VS + 2 * e));
-      a0 = fmaf(p, v.x, a0);
-      a1 = fmaf(p, v.y, a1);
-    }
-  }
-  a0 = lanes::reduce<S::KQ>(a0, lanes::Add{});
-  a1 = lanes::reduce<S::KQ>(a1, lanes::Add{});
-  if (kq == 0 && oe < GROUP * PAIRS)
-    *(float2*)(part_acc + (slot0 + (int64_t)g * max_chunks + c) * D + 2 * e) = make_float2(a0, a1);
-}
-
-// attend_mfma_kernel: the same slice as attend_wide_kernel (one 64-key
-// slice x one key head x one token, f16 cache, GROUP <= 4 query heads of
-// head_dim D), with both products on the matrix cores
-// (v_mfma_f32_16x16x32_f16), as attend_flash.hip computes them for a
-// prefill chunk.  At 4 and 8 sequences the VALU dot loops of the wide
-// kernel bound its time; here a block of 256 threads does
-//   * S = K Q^T: wave w takes keys 16w..16w+15 as the A rows, read straight
-//     from the cache into fragments; the N columns are the GROUP queries as
-//     three halves each (q1 = f16(q), q2 = f16(q - q1), q3 = f16(q - q1 -
-//     q2): every bit of the f32 query), staged once in LDS, so a score is
-//     the sum of three columns;
-//   * the slice softmax, one wave per query head (lane = key), as the wide
-//     kernel;
-//   * O = P V: P as two halves (rows h and GROUP + h), V staged by rows
-//     (exact halves); wave w takes D / 64 of the D / 16 column tiles.
-// MFMA fragments (16x16x32): lane l holds row / column l % 16 and values
-// 8 (l / 16) .. +8 of the 32; result element i of lane l is row 4 (l / 16)
-// + i, column l % 16.  The partial sums land where attend_wide_kernel
-// writes them.
-// PAGED: kv_index maps positions to cache cells; without it the cell is
-// the position, and no index load sits under a branch (which would make the
-// compiler wait for every load in flight at the join: the keys before the
-// values went out).
-template <int GROUP, int D, bool PAGED>
-__global__ __launch_bounds__(256) void attend_mfma_kernel(
-    const float* __restrict__ q, int64_t q_stride, const __half* __restrict__ kc, const __half* __restrict__ vc,
-    int64_t cache_stride, int heads, int kv_heads, float scale, const int32_t* __restrict__ pos_dev,
-    int count_host, int max_chunks, float* __restrict__ part_acc, float* __restrict__ part_ml,
-    const int32_t* __restrict__ kv_index_arg, int64_t index_stride) {
-  const int32_t* __restrict__ kv_index = PAGED ? kv_index_arg : nullptr;
-  static_assert(GROUP == 1 || GROUP == 2 || GROUP == 4, "three halves of GROUP queries fill at most 12 columns");
-  static_assert(D == 64 || D == 128, "head_dim 64 or 128");
-  constexpr int KK = kWideKeys, QP = D + 8, KP = KK + 8;
-  constexpr int PIECES = D / 8, PER = KK * PIECES / 256;
-  __shared__ __align__(16) _Float16 Qh[3 * GROUP * QP];
-  __shared__ __align__(16) _Float16 Vr[KK * QP];
-  __shared__ __align__(16) _Float16 Ph[2 * GROUP * KP];
-  __shared__ float Ss[GROUP * KK];
-  const int c = blockIdx.x, kvh = blockIdx.y, t = blockIdx.z;
-  const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
-  const int lm = lane & 15, lk = lane >> 4;
-  const int count = pos_dev ? pos_dev[t] + 1 : count_host;
-  const int start = c * KK;
-  if (start >= count) return;
-  const int nk = min(KK, count - start);
-  const int kvw = kv_heads * D;
-  const int64_t seq = kv_index ? 0 : (int64_t)t * cache_stride;
-
-  // this wave's 16 keys as A fragments (key 16 wave + lm, values 32 ks +
-  // 8 lk .. +8), the block's share of the values, and the queries; keys past
-  // the end repeat the last live one (masked below)
-  const __half* kb = kc + seq + (int64_t)kvh * D;
-  const __half* vb = vc + seq + (int64_t)kvh * D;
-  // the queries first, then the keys, then the values: loads complete in
-  // issue order, so the query halves wait only for the queries and the
-  // scores only for the keys, while the values are still arriving
-  constexpr int NQ4 = GROUP * D / 4;
-  const float* qg = q + (int64_t)t * q_stride + (int64_t)kvh * GROUP * D;
-  const att_f4 qv = ((const att_f4*)qg)[tid < NQ4 ? tid : 0];
-  __builtin_amdgcn_sched_barrier(0);
-  att_h8 ka[D / 32];
-  {
-    const int cell = max(kv_cell(kv_index, index_stride, t, start + min(16 * wave + lm, nk - 1)), 0);
-#pragma unroll
-    for (int ks = 0; ks < D / 32; ks++) ka[ks] = *(const att_h8*)(kb + (int64_t)cell * kvw + 32 * ks + 8 * lk);
-  }
-  // (native vectors: an array of HIP's uint4 struct went to scratch)
-  att_h8 vraw[PER];
-#pragma unroll
-  for (int j = 0; j < PER; j++) {
-    const int i = tid + j * 256;
-    const int key = i / PIECES, pc = i % PIECES;
-    const int cell = max(kv_cell(kv_index, index_stride, t, start + min(key, nk - 1)), 0);
-    vraw[j] = *(const att_h8*)(vb + (int64_t)cell * kvw + pc * 8);
-  }
-  __builtin_amdgcn_sched_barrier(0);
-  {
-    // query h = tid / (D / 4), dims 4 (tid % (D / 4)) .. +4, as three halves
-    // (computed by every thread, so the query load is not sunk into the
-    // branch behind the keys and values; threads past NQ4 store nothing)
-    const int h = (tid < NQ4 ? tid : 0) / (D / 4), d0 = 4 * ((tid < NQ4 ? tid : 0) % (D / 4));
-    float qf[4] = {qv.x, qv.y, qv.z, qv.w};
-    // here, not inside the branch below (where the compiler would sink the
-    // query load, behind the keys and values)
-    asm volatile("" : "+v"(qf[0]), "+v"(qf[1]), "+v"(qf[2]), "+v"(qf[3]));
-    _Float16 hv[3][4];
-#pragma unroll
-    for (int u = 0; u < 4; u++) {
-      const _Float16 h1 = (_Float16)qf[u];
-      const float r1 = qf[u] - (float)h1;  // exact
-      const _Float16 h2 = (_Float16)r1;
-      hv[0][u] = h1;
-      hv[1][u] = h2;
-      hv[2][u] = (_Float16)(r1 - (float)h2);
-    }
-    if (tid < NQ4) {
-#pragma unroll
-      for (int k = 0; k < 3; k++)
-#pragma unroll
-        for (int u = 0; u < 4; u++) Qh[(k * GROUP + h) * QP + d0 + u] = hv[k][u];
-    }
-  }
-  __syncthreads();
-
-  // S for keys 16 wave .. +15 against column lm = (half lm / GROUP, query
-  // lm % GROUP); columns from 3 GROUP on are zero
-  {
-    att_f4 sacc = att_f4{0.0f, 0.0f, 0.0f, 0.0f};
-    const bool qcol = lm < 3 * GROUP;
-    const int qrow = qcol ? lm : 0;
-#pragma unroll
-    for (int ks = 0; ks < D / 32; ks++) {
-      const att_h8 qb = *(const att_h8*)(Qh + qrow * QP + 32 * ks + 8 * lk);
-      sacc = att_mfma(ka[ks], qcol ? qb : att_h8{0, 0, 0, 0, 0, 0, 0, 0}, sacc);
-    }
-    // lanes lm < GROUP: the score of query lm at keys 16 wave + 4 lk + i,
-    // its three halves added in order
-#pragma unroll
-    for (int i = 0; i < 4; i++) {
-      // (row shifts within the lane's 16-lane row: lanes lm < GROUP read
-      // lm + GROUP and lm + 2 GROUP)
-      const float s2 = __uint_as_float(lanes::dpp<0x100 + GROUP>(__float_as_uint(sacc[i])));
-      const float s3 = __uint_as_float(lanes::dpp<0x100 + 2 * GROUP>(__float_as_uint(sacc[i])));
-      const float sc = (sacc[i] + s2) + s3;
-      const int key = 16 * wave + 4 * lk + i;
-      const bool live = key < nk && (!kv_index || kv_cell(kv_index, index_stride, t, start + key) >= 0);
-      if (lm < GROUP) Ss[lm * KK + key] = live ? sc * scale : -INFINITY;
-    }
-  }
-  // the values into LDS once the scores are out (they are read after the
-  // softmax barrier)
-#pragma unroll
-  for (int j = 0; j < PER; j++) {
-    const int i = tid + j * 256;
-    const int key = i / PIECES, pc = i % PIECES;
-    *(att_h8*)(Vr + key * QP + pc * 8) = vraw[j];
-  }
-  __syncthreads();
-  const int64_t slot0 = ((int64_t)t * heads + (int64_t)kvh * GROUP) * max_chunks;
-  // slice softmax: wave g takes query g, lane = key; P as two halves
-  if (wave < GROUP) {
-    const float sc = Ss[wave * KK + lane];
-    const float m = lanes::reduce<64>(sc, lanes::Max{});
-    const float pr = sc == -INFINITY ? 0.0f : expf(sc - m);
-    const float l = lanes::reduce<64>(pr, lanes::Add{});
-    // P lifted by 2^14 (exact; p <= 1 stays below the largest half) so that
-    // the low halves of small weights are not f16 subnormals
-    const float pl = pr * kPLift;
-    const _Float16 ph = (_Float16)pl;
-    Ph[wave * KP + lane] = ph;
-    Ph[(GROUP + wave) * KP + lane] = (_Float16)(pl - (float)ph);
-    if (lane == 0) *(float2*)(part_ml + (slot0 + (int64_t)wave * max_chunks + c) * 2) = make_float2(m, l);
-  }
-  __syncthreads();
-  // O for column tiles nt = wave, wave + 4, ...: rows (half, query) =
-  // 4 lk + i, column = dim 16 nt + lm; rows from 2 GROUP on are zero
-  {
-    const bool prow = lm < 2 * GROUP;
-    const int arow = prow ? lm : 0;
-    att_h8 pa[KK / 32];
-#pragma unroll
-    for (int ks = 0; ks < KK / 32; ks++) {
-      const att_h8 a = *(const att_h8*)(Ph + arow * KP + 32 * ks + 8 * lk);
-      pa[ks] = prow ? a : att_h8{0, 0, 0, 0, 0, 0, 0, 0};
-    }
-#pragma unroll
-    for (int nt = wave; nt < D / 16; nt += 4) {
-      att_f4 oacc = att_f4{0.0f, 0.0f, 0.0f, 0.0f};
-#pragma unroll
-      for (int ks = 0; ks < KK / 32; ks++)
-      {
-        // the B fragment (dim 16 nt + lm, keys 32 ks + 8 lk .. +8) gathered
-        // from the row-major values: staging them transposed (a 2-byte
-        // store per value, 8-way bank conflicts) took the kernel from 10.5
-        // to 17.9 us at 4 sequences
-        att_h8 vb;
-#pragma unroll
-        for (int e = 0; e < 8; e++) vb[e] = Vr[(32 * ks + 8 * lk + e) * QP + 16 * nt + lm];
-        oacc = att_mfma(pa[ks], vb, oacc);
-      }
-      const int dim = 16 * nt + lm;
-      // query g's output: row g (hi) plus row GROUP + g (lo)
-      if constexpr (GROUP == 4) {
-        // rows 0..3 in lanes lk = 0, rows 4..7 in lanes lk = 1
-#pragma unroll
-        for (int i = 0; i < 4; i++) {
-          // row 0 (lk = 0) and row 1 swapped across: p[1] of a row-0 lane is
-          // its row-1 partner's value
-          const auto p = __builtin_amdgcn_permlane16_swap(__float_as_uint(oacc[i]), __float_as_uint(oacc[i]), false,
-                                                          false);
-          const float hi = __uint_as_float(p[0]), lo = __uint_as_float(p[1]);
-          if (lk == 0) part_acc[(slot0 + (int64_t)i * max_chunks + c) * D + dim] = (hi + lo) * kPDrop;
-        }
-      } else if constexpr (GROUP == 2) {
-        if (lk == 0) {
-          part_acc[(slot0 + 0 * (int64_t)max_chunks + c) * D + dim] = (oacc[0] + oacc[2]) * kPDrop;
-          part_acc[(slot0 + 1 * (int64_t)max_chunks + c) * D + dim] = (oacc[1] + oacc[3]) * kPDrop;
-        }
-      } else {
-        if (lk == 0) part_acc[(slot0 + c) * D + dim] = (oacc[0] + oacc[1]) * kPDrop;
-      }
-    }
-  }
-}
-
-// attend_wide_q8_kernel: attend_wide_kernel over a q8_0 cache (the row's
-// quants of every key head, then its factors: cache_row), the arithmetic of
-// attend_split_q8_kernel (each key or value element float(quant) *
-// float(factor) before it is used) spread the same way as the f16 form:
-// a score is SPL threads of DPT dims (whole 32-value blocks, so one factor a
-// block), a weighted value pair is KQ threads over interleaved keys, and the
-// slice softmax is one wave per query head.
-template <int GROUP, int D, int NT>
-__global__ __launch_bounds__(NT) void attend_wide_q8_kernel(
-    const float* __restrict__ q, int64_t q_stride, const __half* __restrict__ kc, const __half* __restrict__ vc,
-    int64_t cache_stride, int row, int heads, int kv_heads, float scale, const int32_t* __restrict__ pos_dev,
-    int count_host, int max_chunks, float* __restrict__ part_acc, float* __restrict__ part_ml,
-    const int32_t* __restrict__ kv_index, int64_t index_stride) {
-#pragma clang fp contract(off)
-  using S = WideShape<GROUP, D, NT>;
-  constexpr int KK = kWideKeys, NB = D / 32, PIECES = D / 16, TOTAL = KK * PIECES, PAIRS = D / 2;
-  constexpr int PER = (TOTAL + NT - 1) / NT;  // 16-byte pieces of K (and of V) per thread
-  constexpr int KQR = D + 16;                 // LDS key rows in bytes (16 bytes of pad)
-  static_assert(GROUP * D / 4 <= NT && S::KQ >= 1 && S::KQ <= 64, "shape");
-  if constexpr (S::DPT % 16 != 0) {
-    return;  // never launched (wide_q8_fits): a score part is whole 16-byte pieces
-  } else {
-  __shared__ __align__(16) int8_t Kq[KK * KQR];
-  __shared__ __align__(16) int8_t Vq[KK * D];
-  __shared__ float Ksc[KK * NB], Vsc[KK * NB];
-  __shared__ __align__(16) float Qs[GROUP * D];
-  __shared__ float Ss[GROUP * KK];
-  const int c = blockIdx.x, kvh = blockIdx.y, t = blockIdx.z;
-  const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
-  const int count = pos_dev ? pos_dev[t] + 1 : count_host;
-  const int start = c * KK;
-  if (start >= count) return;
-  const int nk = min(KK, count - start);
-  const int kvw = kv_heads * D;
-
-  const float* qg = q + (int64_t)t * q_stride + (int64_t)kvh * GROUP * D;
-  const bool has_q = tid < GROUP * D / 4;
-  const float4 qv = ((const float4*)qg)[has_q ? tid : 0];
-  const int64_t seq = kv_index ? 0 : (int64_t)t * cache_stride;
-  const int8_t* kseq = (const int8_t*)(kc + seq);
-  const int8_t* vseq = (const int8_t*)(vc + seq);
-  uint4 kraw[PER], vraw[PER];
-#pragma unroll
-  for (int j = 0; j < PER; j++) {
-    const int i = min(tid + j * NT, TOTAL - 1);
-    const int key = i / PIECES, pc = i % PIECES;
-    const int cell = max(kv_cell(kv_index, index_stride, t, start + min(key, nk - 1)), 0);
-    const int64_t off = (int64_t)cell * row * 2 + (int64_t)kvh * D + pc * 16;  // bytes
-    kraw[j] = *(const uint4*)(kseq + off);
-    vraw[j] = *(const uint4*)(vseq + off);
-  }
-  // the factors: KK * NB of each, at most one of each a thread
-  const bool has_f = tid < KK * NB;
-  float kf = 0.0f, vf = 0.0f;
-  {
-    const int i = has_f ? tid : 0, key = i / NB, b = i % NB;
-    const int cell = max(kv_cell(kv_index, index_stride, t, start + min(key, nk - 1)), 0);
-    const int64_t at = (int64_t)cell * row + (kvw >> 1) + (kvh * D >> 5) + b;  // halves
-    kf = __half2float(kc[seq + at]);
-    vf = __half2float(vc[seq + at]);
-  }
-  if (has_q) ((float4*)Qs)[tid] = qv;
-  if (has_f) {
-    Ksc[tid] = kf;
-    Vsc[tid] = vf;
-  }
-#pragma unroll
-  for (int j = 0; j < PER; j++) {
-    const int i = tid + j * NT;
-    const int key = i / PIECES, pc = i % PIECES;
-    if (i < TOTAL) {
-      *(uint4*)(Kq + key * KQR + pc * 16) = kraw[j];
-      *(uint4*)(Vq + key * D + pc * 16) = vraw[j];
-    }
-  }
-  __syncthreads();
-
-  // scores: thread = (query head g, key, part of DPT dims)
-  {
-    const int dot = tid / S::SPL, part = tid % S::SPL;
-    const int g = dot / KK, key = dot % KK;
-    float sdot = 0.0f;
-    if (dot < GROUP * KK) {
-      const int8_t* kr = Kq + key * KQR + part * S::DPT;
-      const float* qq = Qs + g * D + part * S::DPT;
-#pragma unroll
-      for (int d = 0; d < S::DPT; d += 16) {
-        const float f = Ksc[key * NB + (part * S::DPT + d) / 32];
-        const uint4 raw = *(const uint4*)(kr + d);
-        const int8_t* b = (const int8_t*)&raw;
-#pragma unroll
-        for (int i = 0; i < 16; i++) sdot = fmaf(qq[d + i], (float)b[i] * f, sdot);
-      }
-    }
-    sdot = lanes::reduce<S::SPL>(sdot, lanes::Add{});
-    if (part == 0 && dot < GROUP * KK) {
-      const bool live = key < nk && (!kv_index || kv_cell(kv_index, index_stride, t, start + key) >= 0);
-      Ss[g * KK + key] = live ? sdot * scale : -INFINITY;
-    }
-  }
-  __syncthreads();
-  const int64_t slot0 = ((int64_t)t * heads + (int64_t)kvh * GROUP) * max_chunks;
-  if (wave < GROUP) {
-    const float sc = Ss[wave * KK + lane];
-    const float m = lanes::reduce<64>(sc, lanes::Max{});
-    const float pr = sc == -INFINITY ? 0.0f : expf(sc - m);
-    const float l = lanes::reduce<64>(pr, lanes::Add{});
-    Ss[wave * KK + lane] = pr;
-    if (lane == 0) *(float2*)(part_ml + (slot0 + (int64_t)wave * max_chunks + c) * 2) = make_float2(m, l);
-  }
-  __syncthreads();
-  // unnormalised weighted values: thread = (query head, dim pair, key residue kq)
-  const int kq = tid % S::KQ, oe = tid / S::KQ;
-  const int g = oe / PAIRS, e = oe % PAIRS;
-  float a0 = 0.0f, a1 = 0.0f;
-  if (oe < GROUP * PAIRS) {
-    const float* pg = Ss + g * KK;
-    const int b = (2 * e) >> 5;
-#pragma unroll 4
-    for (int k = kq; k < KK; k += S::KQ) {
-      const float p = pg[k];
-      const char2 v = *(const char2*)(Vq + k * D + 2 * e);
-      const float f = Vsc[k * NB + b];
-      a0 = fmaf(p, (float)v.x * f, a0);
-      a1 = fmaf(p, (float)v.y * f, a1);
-    }
-  }
-  a0 = lanes::reduce<S::KQ>(a0, lanes::Add{});
-  a1 = lanes::reduce<S::KQ>(a1, lanes::Add{});
-  if (kq == 0 && oe < GROUP * PAIRS)
-    *(float2*)(part_acc + (slot0 + (int64_t)g * max_chunks + c) * D + 2 * e) = make_float2(a0, a1);
-  }
-}
-
-// whether attend_wide_q8_kernel takes a shape: each score thread's dims are
-// whole 16-byte pieces
-__host__ __device__ constexpr bool wide_q8_fits(int group, int d, int nt) {
-  return d % (16 * (nt / (group * kWideKeys) < d / 8 ? nt / (group * kWideKeys) : d / 8)) == 0;
 }
 
 // ---- the optional layer parts of other families ----------------------------
@@ -1510,11 +1012,15 @@ int launch_store_kv(hipStream_t s, const float* k, const float* v, int32_t kv_wi
 // attend_merge_kernel with B the slice count rounded up to 8 (at most 64)
 static int launch_merge(hipStream_t s, const float* part_acc, const float* part_ml, int heads, int head_dim,
                         const int32_t* pos_dev, int count_host, int chunks, int tokens, float* out, void* xq_out,
-                        void* hx_out) {
+                        void* hx_out, bool fold = false) {
   const dim3 grid(heads, tokens), block(head_dim < 64 ? 64 : head_dim);
-#define MI_MERGE(B)                                                                                    \
-  hipLaunchKernelGGL(attend_merge_kernel<B>, grid, block, 0, s, part_acc, part_ml, heads, head_dim, pos_dev, \
-                     count_host, chunks, out, (uint8_t*)xq_out, (uint8_t*)hx_out)
+#define MI_MERGE(B)                                                                                            \
+  if (fold)                                                                                                    \
+    hipLaunchKernelGGL((attend_merge_kernel<B, true>), grid, block, 0, s, part_acc, part_ml, heads, head_dim,    \
+                       pos_dev, count_host, chunks, out, (uint8_t*)xq_out, (uint8_t*)hx_out);                    \
+  else                                                                                                         \
+    hipLaunchKernelGGL((attend_merge_kernel<B, false>), grid, block, 0, s, part_acc, part_ml, heads, head_dim,   \
+                       pos_dev, count_host, chunks, out, (uint8_t*)xq_out, (uint8_t*)hx_out)
   switch ((std::min(chunks, 64) + 7) / 8) {
     case 1: MI_MERGE(8); break;
     case 2: MI_MERGE(16); break;
@@ -1549,53 +1055,16 @@ int launch_attend(hipStream_t s, const float* q, int64_t q_stride, const uint16_
   const size_t acc_bytes = ((size_t)slots * head_dim * sizeof(float) + 255) & ~(size_t)255;
   float* part_ml = (float*)((char*)work + acc_bytes);
   const int group = heads / kv_heads;
-  // decode (at most 8 tokens, one each per sequence): the matrix-core slice
-  // kernel for an f16 cache and up to 4 query heads a key head, else the
-  // wide VALU slice kernel (1024 threads at one token, 512 for a batch)
-  if (tokens <= kMaxTokens && (head_dim == 64 || head_dim == 128) &&
-      (form != MI_CACHE_Q8 || wide_q8_fits(group, head_dim, tokens == 1 ? 1024 : 512))) {
-    dim3 grid(chunks, kv_heads, tokens);
-    const int qrow = cache_row(MI_CACHE_Q8, kv_heads * head_dim);
-#define MI_WIDE(G, DD)                                                                                       \
-  if (form == MI_CACHE_Q8 && tokens == 1)                                                                    \
-    hipLaunchKernelGGL((attend_wide_q8_kernel<G, DD, 1024>), grid, dim3(1024), 0, s, q, q_stride,            \
-                       (const __half*)k_cache, (const __half*)v_cache, cache_stride, qrow, heads, kv_heads,   \
-                       scale, pos_dev, count_host, chunks, part_acc, part_ml, kv_index, index_stride);        \
-  else if (form == MI_CACHE_Q8)                                                                              \
-    hipLaunchKernelGGL((attend_wide_q8_kernel<G, DD, 512>), grid, dim3(512), 0, s, q, q_stride,              \
-                       (const __half*)k_cache, (const __half*)v_cache, cache_stride, qrow, heads, kv_heads,   \
-                       scale, pos_dev, count_host, chunks, part_acc, part_ml, kv_index, index_stride);        \
-  else if (G <= 4 && kv_index)                                                                               \
-    hipLaunchKernelGGL((attend_mfma_kernel<(G <= 4 ? G : 4), DD, true>), grid, dim3(256), 0, s, q, q_stride,  \
-                       (const __half*)k_cache, (const __half*)v_cache, cache_stride, heads, kv_heads, scale,   \
-                       pos_dev, count_host, chunks, part_acc, part_ml, kv_index, index_stride);               \
-  else if (G <= 4)                                                                                           \
-    hipLaunchKernelGGL((attend_mfma_kernel<(G <= 4 ? G : 4), DD, false>), grid, dim3(256), 0, s, q, q_stride, \
-                       (const __half*)k_cache, (const __half*)v_cache, cache_stride, heads, kv_heads, scale,   \
-                       pos_dev, count_host, chunks, part_acc, part_ml, kv_index, index_stride);               \
-  else if (tokens == 1)                                                                                      \
-    hipLaunchKernelGGL((attend_wide_kernel<G, DD, 1024>), grid, dim3(1024), 0, s, q, q_stride,               \
-                       (const __half*)k_cache, (const __half*)v_cache, cache_stride, heads, kv_heads, scale,   \
-                       pos_dev, count_host, chunks, part_acc, part_ml, kv_index, index_stride);               \
-  else                                                                                                       \
-    hipLaunchKernelGGL((attend_wide_kernel<G, DD, 512>), grid, dim3(512), 0, s, q, q_stride,                 \
-                       (const __half*)k_cache, (const __half*)v_cache, cache_stride, heads, kv_heads, scale,   \
-                       pos_dev, count_host, chunks, part_acc, part_ml, kv_index, index_stride)
-#define MI_WIDE_D(G) \
-  if (head_dim == 64) { MI_WIDE(G, 64); } else { MI_WIDE(G, 128); }
-    switch (group) {
-      case 1: MI_WIDE_D(1); break;
-      case 2: MI_WIDE_D(2); break;
-      case 4: MI_WIDE_D(4); break;
-      case 8: MI_WIDE_D(8); break;
-      default: return fail(MI_ERR_SHAPE, "attend: %d query heads per key head is not 1, 2, 4 or 8", group);
-    }
-#undef MI_WIDE_D
-#undef MI_WIDE
-    int rc = hip_check(hipGetLastError(), "attend_wide launch");
-    if (rc) return rc;
-    return launch_merge(s, part_acc, part_ml, heads, head_dim, pos_dev, count_host, chunks, tokens, out, xq_out,
-                        hx_out);
+  // decode (at most 8 tokens, one each per sequence): shares of the keys, then
+  // their fold
+  if (tokens <= kMaxTokens && decode_attend_fits(group, head_dim)) {
+    const int shares = decode_attend_shares(kv_heads, tokens, max_count);
+    if (int rc = launch_attend_decode(s, q, q_stride, k_cache, v_cache, cache_stride, heads, kv_heads, head_dim, scale,
+                                      pos_dev, count_host, shares, tokens, part_acc, part_ml, form, kv_index,
+                                      index_stride))
+      return rc;
+    return launch_merge(s, part_acc, part_ml, heads, head_dim, pos_dev, count_host, shares, tokens, out, xq_out, hx_out,
+                        true);
   }
   // one sequence's chunk (its tokens share one cache): the flash kernel at head
   // widths 64 and 128, else 16 tokens per block over one staged slice (f16

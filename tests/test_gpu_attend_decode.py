@@ -1,0 +1,71 @@
+"""Decode attention (attend_decode.hip) at the sizes where it can go wrong:
+counts around a wave's 32-key run, a block's 128-key step and past 64 steps (a
+share of two), every group size and both head widths over both cache forms, a
+context far longer than the position (shares without keys), and a workspace
+that held NaN before (those shares' values are never written).  Gate: 1e-5 of
+the peak against the oracle, as tests/test_gpu_kernels.py test_attention.
+"""
+
+import numpy as np
+import pytest
+import torch
+
+import oracle
+from molla_amd import synth
+
+pytestmark = pytest.mark.gpu
+
+
+def caches(form, count, kvw, seed):
+    from tests.test_gpu_kernels import q8_decode, q8_rows
+    dev, host = [], []
+    for i in (0, 1):
+        raw = synth.normal(count * kvw, seed + i).numpy()
+        h = q8_rows(raw, kvw) if form == "q8" else raw.astype(np.float16).view(np.uint16)
+        dev.append(torch.from_numpy(h.view(np.int16).copy()).view(torch.float16).cuda())
+        host.append(q8_decode(h, kvw, count).reshape(-1) if form == "q8" else h.view(np.float16).astype(np.float32))
+    return dev, host
+
+
+@pytest.mark.parametrize("form", ["f16", "q8"])
+@pytest.mark.parametrize("heads,kv,hd", [(2, 2, 128), (4, 2, 64), (8, 2, 128), (8, 1, 64), (16, 2, 128)])
+@pytest.mark.parametrize("count", [1, 31, 32, 33, 128, 129, 8193])
+def test_decode_attention_edges(form, heads, kv, hd, count):
+    from molla_amd import gpu
+    ctx = gpu.DeviceContext(0)
+    (kd, vd), (kh, vh) = caches(form, count, kv * hd, 40)
+    q = synth.normal(heads * hd, 42).numpy()
+    scale = float(np.float32(1 / np.sqrt(hd)))
+    out = torch.zeros(heads * hd, device="cuda")
+    f = gpu.CACHE_Q8 if form == "q8" else gpu.CACHE_F16
+    gpu.device_attend(ctx, torch.from_numpy(q).cuda(), kd, vd, heads, kv, hd, scale, count, out, f)
+    want = oracle.attend(heads, kv, hd, scale, q, kh, vh, count)
+    assert np.abs(out.cpu().numpy() - want).max() <= 1e-5 * np.abs(want).max()
+
+
+@pytest.mark.parametrize("form", ["f16", "q8"])
+@pytest.mark.parametrize("tokens", [1, 3])
+def test_context_longer_than_the_position(form, tokens):
+    """The shares are cut by the context and filled by the position: the layer
+    over a context of 5000 gives the layer over one of pos + 1 within the
+    rounding of differently grouped sums (1e-6 of each element's own bound
+    would be tests/layer64.py's gate a hundred times over)."""
+    from molla_amd import block, gpu
+    from tests.test_gpu_layer import device_layer_from, make_layer_weights, spec_of
+    ctx = gpu.DeviceContext(0)
+    f = gpu.CACHE_Q8 if form == "q8" else gpu.CACHE_F16
+    bs, layer = device_layer_from(make_layer_weights(spec_of(512, 512, 8, 2, 64), 31), spec_of(512, 512, 8, 2, 64))
+    kvw, pos, ctx_len = bs.kv_width(), 140, 5000
+    row = gpu.cache_row(f, kvw)
+    (k, v), _ = caches(form, tokens * ctx_len, kvw, 50)
+    x = synth.normal(tokens * bs.width, 52).cuda()
+    posd = torch.tensor([pos - 60 * t for t in range(tokens)], dtype=torch.int32, device="cuda")
+    outs = []
+    for max_count in (pos + 1, ctx_len):
+        work = torch.empty(block.layer_workspace(layer, max_count, tokens), dtype=torch.uint8, device="cuda")
+        work.fill_(255)  # NaN as floats
+        xd, kd, vd = x.clone(), k.clone(), v.clone()
+        block.device_layer(ctx, layer, xd, kd, vd, ctx_len * row, posd, max_count, tokens, work=work, form=f)
+        outs.append(xd.cpu().double())
+    assert torch.isfinite(outs[1]).all()
+    assert (outs[0] - outs[1]).norm() <= 1e-5 * outs[0].norm()
