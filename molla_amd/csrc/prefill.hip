@@ -67,7 +67,7 @@ __device__ __forceinline__ v16f mfma(v8h a, v8h b, v16f c) {
 }
 
 __device__ __forceinline__ v8h as_v8h4(v4u u) { return __builtin_bit_cast(v8h, u); }
-// 16 bytes from a 2-byte aligned address (the 34/18/22/210-byte blocks), one
+// 16 bytes from a 2-byte aligned address (Q6_K's 210-byte superblocks), one
 // load: the memory path takes any alignment of whole bytes here.
 typedef uint32_t v4u_a2 __attribute__((ext_vector_type(4), aligned(2)));
 typedef uint32_t u32_a2 __attribute__((aligned(2)));
@@ -273,29 +273,70 @@ struct KB32 {
   // u of the magic halves is the unsigned code; the signed one is u - BIAS
   static constexpr float BIAS = KIND == MI_Q8_0 ? 128.0f : KIND == MI_Q4_0 ? 8.0f : KIND == MI_Q5_0 ? 16.0f : 0.0f;
   static constexpr bool FIVE = KIND == MI_Q5_0 || KIND == MI_Q5_1;
-  static constexpr int QAT = BLOCK - (KIND == MI_Q8_0 ? 32 : 16);
+  // A stage is two blocks, for the kinds of 34, 18 and 22 bytes a whole number
+  // of dwords: they are read from its start, so that on 4-byte aligned weights
+  // every load is aligned, and the first block's codes, two bytes off, are
+  // moved into place.  (The loads take 2-byte alignment too.  Read at the
+  // codes themselves, half of them two bytes off, Q4_0 4096x14336 at 4 tokens
+  // took 39 us against 27.)
+  static constexpr int WORDS = KIND == MI_Q4_0 ? 9 : KIND == MI_Q5_0 ? 11 : KIND == MI_Q8_0 ? 11 : 8 + 2 * (BLOCK - 16) / 4;
+  typedef uint32_t v2u_a2 __attribute__((ext_vector_type(2), aligned(2)));
   struct Raw {
-    uint32_t dm[2];  // d | m << 16
-    uint32_t qh[FIVE ? 2 : 1];
-    v4u q[2];        // [block] the lane's 16 bytes
+    uint32_t w[WORDS];
   };
   typedef NoHdr Hdr;
-  static __device__ __forceinline__ void load(Raw& r, const uint8_t* row, int st, int kh) {
+  static __device__ __forceinline__ void put4(uint32_t* w, const uint8_t* p) {
+    const v4u v = *(const v4u_a2*)p;
 #pragma unroll
-    for (int bb = 0; bb < 2; bb++) {
-      const uint8_t* b = row + (int64_t)(2 * st + bb) * BLOCK;
-      r.dm[bb] = MIN == 2 ? *(const uint32_t*)b : ld2(b);
-      if constexpr (FIVE) r.qh[bb] = ld4u(b + (KIND == MI_Q5_0 ? 2 : 4));
-      r.q[bb] = ld16(b + QAT + (KIND == MI_Q8_0 ? 16 * kh : 0));
+    for (int i = 0; i < 4; i++) w[i] = v[i];
+  }
+  static __device__ __forceinline__ void load(Raw& r, const uint8_t* row, int st, int kh) {
+    const uint8_t* b = row + (int64_t)st * (2 * BLOCK);
+    if constexpr (KIND == MI_Q4_0) {  // d0 q0 | q0 d1 | q1
+      put4(r.w, b);
+      r.w[4] = ld4u(b + 16);
+      put4(r.w + 5, b + 20);
+    } else if constexpr (KIND == MI_Q5_0) {  // d0 h0 q0 d1 | h1 q1
+      put4(r.w, b);
+      put4(r.w + 4, b + 16);
+      const v2u_a2 v = *(const v2u_a2*)(b + 32);
+      r.w[8] = v.x, r.w[9] = v.y;
+      r.w[10] = ld4u(b + 40);
+    } else if constexpr (KIND == MI_Q8_0) {  // half wave kh's 16 bytes of each block, and the two scales
+      put4(r.w, b + 16 * kh);
+      r.w[4] = ld4u(b + 16 + 16 * kh);
+      put4(r.w + 5, b + 36 + 16 * kh);
+      r.w[9] = ld4u(b);
+      r.w[10] = ld4u(b + 32);
+    } else {  // each block: d m [h] q, all aligned
+#pragma unroll
+      for (int bb = 0; bb < 2; bb++) {
+        uint32_t* w = r.w + bb * (WORDS / 2);
+        w[0] = *(const uint32_t*)(b + bb * BLOCK);
+        if constexpr (FIVE) w[1] = *(const uint32_t*)(b + bb * BLOCK + 4);
+        put4(w + WORDS / 2 - 4, b + bb * BLOCK + BLOCK - 16);
+      }
     }
   }
   static __device__ __forceinline__ void load_hdr(Hdr&, const uint8_t*, int, int) {}
+  static __device__ __forceinline__ uint32_t off2(const Raw& r, int i) {  // the dword two bytes into w[i]
+    return __builtin_amdgcn_alignbyte(r.w[i + 1], r.w[i], 2);
+  }
+  // dword i of block bb's codes
+  static __device__ __forceinline__ uint32_t code(const Raw& r, int bb, int i) {
+    if constexpr (KIND == MI_Q4_0 || KIND == MI_Q8_0) return bb ? r.w[5 + i] : off2(r, i);
+    else if constexpr (KIND == MI_Q5_0) return bb ? r.w[7 + i] : off2(r, 1 + i);
+    else return r.w[bb * (WORDS / 2) + WORDS / 2 - 4 + i];
+  }
+  static __device__ __forceinline__ uint32_t fifth(const Raw& r, int bb) {
+    return KIND == MI_Q5_0 ? (bb ? r.w[6] : off2(r, 0)) : r.w[bb * (WORDS / 2) + 1];
+  }
   static __device__ __forceinline__ void codes(const Raw& r, const Hdr&, int, int s4, int kh, v8h& b0, v8h&) {
     const int bb = s4 >> 1, a = s4 & 1;
     v4u p;
 #pragma unroll
     for (int w = 0; w < 2; w++) {
-      uint32_t x = r.q[bb][2 * a + w];
+      uint32_t x = code(r, bb, 2 * a + w);
       if constexpr (KIND == MI_Q8_0) {
         x ^= 0x80808080u;  // int8 + 128
         p[2 * w] = __builtin_amdgcn_perm(0x64646464u, x, 0x04020400u);
@@ -306,7 +347,7 @@ struct KB32 {
         p[2 * w + 1] = pair(x >> 8, kLow);
         if constexpr (FIVE) {
           // bits 0, 2 (1, 3) of the dword's four to bits 4 and 20
-          const uint32_t f = (r.qh[bb] >> (16 * kh)) >> (8 * a + 4 * w);
+          const uint32_t f = (fifth(r, bb) >> (16 * kh)) >> (8 * a + 4 * w);
           p[2 * w] |= ((f & 5u) * 0x40010u) & 0x00100010u;
           p[2 * w + 1] |= (((f >> 1) & 5u) * 0x40010u) & 0x00100010u;
         }
@@ -314,8 +355,13 @@ struct KB32 {
     }
     b0 = offset(p, splat2(-1024.0f - BIAS));
   }
-  static __device__ __forceinline__ float d(const Raw& r, int bb) { return f16f(r.dm[bb]); }
-  static __device__ __forceinline__ uint32_t mbits(const Raw& r, int bb) { return r.dm[bb] >> 16; }
+  static __device__ __forceinline__ float d(const Raw& r, int bb) {
+    if constexpr (KIND == MI_Q4_0) return f16f(bb ? r.w[4] >> 16 : r.w[0]);
+    else if constexpr (KIND == MI_Q5_0) return f16f(bb ? r.w[5] >> 16 : r.w[0]);
+    else if constexpr (KIND == MI_Q8_0) return f16f(bb ? r.w[10] >> 16 : r.w[9]);
+    else return f16f(r.w[bb * (WORDS / 2)]);
+  }
+  static __device__ __forceinline__ uint32_t mbits(const Raw& r, int bb) { return r.w[bb * (WORDS / 2)] >> 16; }
   // (the K-quants' end of a superblock, which never runs for these)
   static __device__ __forceinline__ float d(const Raw&, const Hdr&) { return 0.0f; }
   static __device__ __forceinline__ float dmin(const Hdr&) { return 0.0f; }
@@ -743,17 +789,15 @@ struct Shape {
   int rt, tt, wr, ks;
   int block_rows() const { return wr * rt * 32; }
 };
-// Each measured against the others (us, with a split's reduce): Q4_K
-// 14336x4096 at 30 tokens 21.1 / 26.9 and Q6_K 4096x14336 at 16 45.5 / 48.7
-// for (1, 1, 4, 4) / (1, 2, 4, 2), but Q8_0 4096x4096 at 20 24.6 / 19.1 (the
-// 32-value kinds' loads are more and smaller: fewer waves wait less);
-// Q4_K 6144x4096 at 256 43.7 / 45.7 and 4096x14336 85.0 / 77.3 for (1, 2, 4, 2) /
-// (2, 2, 4, 2): small matrices want more, smaller blocks; Q6_K 4096x14336 at
-// 256 112 / 121 / 135 for (1, 4, 8, 1) / (1, 4, 4, 1) / (2, 2, 4, 2), its three
-// products a step paying for the larger token tile.
+// Each measured against the others (us, with a split's reduce): up to 32 tokens
+// (1, 1, 4, 2) / (1, 2, 4, 2) / (1, 1, 4, 4): Q4_K 4096x4096 12.7 / 13.8 / 13.5,
+// Q6_K 17.2 / - / 22.9, Q8_0 17.7 / 19.1 / 24.6; Q4_K 6144x4096 at 256 43.7 /
+// 45.7 and 4096x14336 85.0 / 77.3 for (1, 2, 4, 2) / (2, 2, 4, 2): small matrices
+// want more, smaller blocks; Q6_K 4096x14336 at 256 112 / 121 / 135 for
+// (1, 4, 8, 1) / (1, 4, 4, 1) / (2, 2, 4, 2), its three products a step paying for
+// the larger token tile.
 Shape shape_for(int kind, int rows, int cols, int tokens) {
-  const bool k_quant = kind == MI_Q4_K || kind == MI_Q5_K || kind == MI_Q6_K;
-  if (tokens <= 32 && k_quant) return Shape{1, 1, 4, 4};
+  if (tokens <= 32) return Shape{1, 1, 4, 2};
   const int64_t work = (int64_t)((rows + 255) / 256) * ((tokens + 63) / 64) * ((cols + kChunk - 1) / kChunk);
   if (work <= 1536) return Shape{1, 2, 4, 2};
   if (kind == MI_Q6_K && tokens > 64) return Shape{1, 4, 8, 1};
@@ -771,13 +815,8 @@ int launch_kind(hipStream_t s, const RowSegs& sg, int cols, int tokens, const vo
 #define MI_PF(R, T, W, G)                                                                                  \
   hipLaunchKernelGGL((prefill_kernel<KIND, R, T, W, G>), grid, block, 0, s, sg, cols, tokens,               \
                      (const uint8_t*)work, cps, y, ldy, epi, aux, splits > 1 ? part : nullptr)
-  if constexpr (KindOf<KIND>::T::GROUP == 256) {
-    if (sh.tt == 1) {
-      MI_PF(1, 1, 4, 4);
-      return hip_check(hipGetLastError(), "prefill launch");
-    }
-  }
-  if (sh.rt == 1 && sh.tt == 2) MI_PF(1, 2, 4, 2);
+  if (sh.tt == 1) MI_PF(1, 1, 4, 2);
+  else if (sh.rt == 1 && sh.tt == 2) MI_PF(1, 2, 4, 2);
   else if constexpr (KIND == MI_Q6_K) {
     if (sh.tt == 4) MI_PF(1, 4, 8, 1);
     else MI_PF(2, 2, 4, 2);
@@ -826,7 +865,7 @@ bool prefill_fits(int kind, int32_t cols, int64_t row_bytes, const void* w) {
 
 size_t prefill_workspace(int32_t rows, int32_t cols, int32_t tokens) {
   const Prep P = prep_layout(cols, tokens);
-  int splits = 1;
+  int splits = 1;  // the most any kind takes (shape_for tells two apart)
   for (int k : {MI_Q4_K, MI_Q6_K}) splits = std::max(splits, rows > 0 ? choose_splits(k, rows, cols, tokens) : 1);
   size_t part = splits > 1 ? (size_t)splits * tokens * rows * 4 : 0;
   return P.total + ((part + 255) & ~(size_t)255);

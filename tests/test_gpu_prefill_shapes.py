@@ -16,7 +16,7 @@ pytestmark = pytest.mark.gpu
 
 SHAPES = [
     # rows, K-quant cols, 32-value cols, tokens
-    (129, 512, 448, 32),      # one token tile, the K-quants' four groups of K
+    (129, 512, 448, 32),      # one token tile, chunks in two groups of K
     (129, 768, 576, 33),      # the small shape, three chunks in two groups
     (257, 1280, 1344, 65),    # its second block of tokens
     (300, 14592, 14400, 897),  # the large shapes: 57 chunks, ragged rows and tokens
