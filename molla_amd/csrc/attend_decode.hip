@@ -218,7 +218,7 @@ __global__ __launch_bounds__(64 * kWaves, 2) void attend_decode_kernel(
   int xo[Q8 ? KS : 1];  // q8_0: the X that each 32-dim block of o is held at
 #pragma unroll
   for (int b = 0; b < (Q8 ? KS : 1); b++) xo[b] = -100;
-  float mc = -1e30f, l = 0.0f;
+  float mc = -1e30f, l = 0.0f;  // the running maximum is of the scores, before c2
 
   for (int sl = s0; sl < s1; sl++, key0 += kStep) {
     if (key0 >= count) break;  // (uniform over the wave: no keys left for it)
@@ -271,9 +271,9 @@ __global__ __launch_bounds__(64 * kWaves, 2) void attend_decode_kernel(
         m = fmaxf(m, s[a][i]);
       }
     m = across(m, lanes::Max{});
-    const float mn = fmaxf(mc, m == -INFINITY ? -1e30f : m * c2);
+    const float mn = fmaxf(mc, m);
     if (__any(mn != mc)) {
-      const float f = __builtin_amdgcn_exp2f(mc - mn);
+      const float f = __builtin_amdgcn_exp2f((mc - mn) * c2);
       l *= f;
 #pragma unroll
       for (int dt = 0; dt < NT; dt++) o[dt] *= f;
@@ -284,7 +284,7 @@ __global__ __launch_bounds__(64 * kWaves, 2) void attend_decode_kernel(
     for (int a = 0; a < 2; a++)
 #pragma unroll
       for (int i = 0; i < 4; i++) {
-        const float e = __builtin_amdgcn_exp2f(fmaf(s[a][i], c2, kLift - mc));
+        const float e = __builtin_amdgcn_exp2f(fmaf(s[a][i] - mc, c2, kLift));  // (as in attend_flash.hip)
         p[4 * a + i] = (mine >> (16 * a + i)) & 1 ? e : 0.0f;
         l += p[4 * a + i];
       }
@@ -375,7 +375,7 @@ __global__ __launch_bounds__(64 * kWaves, 2) void attend_decode_kernel(
       *(df4*)(wo + (wave * group + lm) * D + 16 * dt + 4 * lk) = o[dt];
     }
     if (lk == 0) {
-      wml[wave][0][lm] = mc;
+      wml[wave][0][lm] = mc * c2;
       wml[wave][1][lm] = l;
     }
   }

@@ -259,7 +259,7 @@ __global__ __launch_bounds__(256, 2) void attend_flash_kernel(
   int xo[NT];  // q8_0: the X that o[dt] is held at
 #pragma unroll
   for (int dt = 0; dt < NT; dt++) xo[dt] = -100;
-  float mc = -1e30f, l = 0.0f;  // running maximum (times c2) and this half wave's sum
+  float mc = -1e30f, l = 0.0f;  // running maximum (of the scores, before c2) and this half wave's sum
 
   // Lane addresses in bytes.  A piece's slot is an exclusive or, and a row
   // starts at a multiple of the piece bits, so piece 2 st + h of this lane's
@@ -342,19 +342,20 @@ __global__ __launch_bounds__(256, 2) void attend_flash_kernel(
 #pragma unroll
     for (int j = 1; j < 16; j++) m = fmaxf(m, s[j]);
     m = other_max(m);
-    const float mn = fmaxf(mc, m == -INFINITY ? -1e30f : m * c2);
+    const float mn = fmaxf(mc, m);
     if (__any(mn != mc)) {
-      const float a = __builtin_amdgcn_exp2f(mc - mn);
+      const float a = __builtin_amdgcn_exp2f((mc - mn) * c2);
       l *= a;
 #pragma unroll
       for (int dt = 0; dt < NT; dt++) o[dt] *= a;
       mc = mn;
     }
-    const float off = kLift - mc;
     fh8 ph[2], pl[2];
 #pragma unroll
     for (int j = 0; j < 16; j++) {
-      float p = __builtin_amdgcn_exp2f(fmaf(s[j], c2, off));
+      // (the difference first: at scores of 1e9 c2 mc is rounded by up to 64,
+      // and a weight taken against it overflows a half)
+      float p = __builtin_amdgcn_exp2f(fmaf(s[j] - mc, c2, kLift));
       if (!full) p = live(j) ? p : 0.0f;
       l += p;
       const _Float16 hi = (_Float16)p;
@@ -428,7 +429,7 @@ __global__ __launch_bounds__(256, 2) void attend_flash_kernel(
       *(ff4*)(dst + 32 * dt + 8 * j4 + 4 * h) = v;
     }
   }
-  if (splits > 1 && h == 0) *(float2*)(part_ml + (rowi * splits + split) * 2) = make_float2(mc, l);
+  if (splits > 1 && h == 0) *(float2*)(part_ml + (rowi * splits + split) * 2) = make_float2(mc * c2, l);
 }
 
 // Folds the splits of each (token, head) row: thread = 4 dims.  A split that

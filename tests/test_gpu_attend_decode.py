@@ -44,6 +44,25 @@ def test_decode_attention_edges(form, heads, kv, hd, count):
 
 
 @pytest.mark.parametrize("form", ["f16", "q8"])
+def test_scores_of_1e8(form):
+    """Scores whose rounding is worth several powers of two of a weight: the
+    largest weight stays 1.  Neighbouring scores lie 1e5 apart and more, so the
+    gate above holds (one key has all the weight)."""
+    from molla_amd import gpu
+    ctx = gpu.DeviceContext(0)
+    heads, kv, hd, count = 8, 2, 128, 300
+    (kd, vd), (kh, vh) = caches(form, count, kv * hd, 60)
+    q = synth.normal(heads * hd, 62).numpy()
+    q *= np.float32(3e4 / np.abs(q).max())
+    scale = np.float32(1e3)
+    out = torch.zeros(heads * hd, device="cuda")
+    f = gpu.CACHE_Q8 if form == "q8" else gpu.CACHE_F16
+    gpu.device_attend(ctx, torch.from_numpy(q).cuda(), kd, vd, heads, kv, hd, float(scale), count, out, f)
+    want = oracle.attend(heads, kv, hd, float(scale), q, kh, vh, count)
+    assert np.abs(out.cpu().numpy() - want).max() <= 1e-5 * np.abs(want).max()
+
+
+@pytest.mark.parametrize("form", ["f16", "q8"])
 @pytest.mark.parametrize("tokens", [1, 3])
 def test_context_longer_than_the_position(form, tokens):
     """The shares are cut by the context and filled by the position: the layer
