@@ -558,8 +558,7 @@ static int llama_layer(hipStream_t s, const mi_layer_desc* d, float* resid, uint
                           d->wv.kind == MI_Q4_K && q4k_tile_fits(d->width, tokens);
     // a Q4_K_M file's layer: Q4_K q and k, Q6_K v
     RowSegs qk{}, vs{};
-    bool mixed_qkv = tokens > 1 && !d->neox && !q8 && d->wq.kind == MI_Q4_K && d->wk.kind == MI_Q4_K &&
-                     d->wv.kind == MI_Q6_K;
+    bool mixed_qkv = tokens > 1 && d->wq.kind == MI_Q4_K && d->wk.kind == MI_Q4_K && d->wv.kind == MI_Q6_K;
     if (mixed_qkv) {
       qk.w[0] = (const uint8_t*)d->wq.data;
       qk.w[1] = qk.w[2] = (const uint8_t*)d->wk.data;
@@ -575,6 +574,16 @@ static int llama_layer(hipStream_t s, const mi_layer_desc* d, float* resid, uint
     if (fused_qkv) {
       // q, k and v in one launch, straight into the fused row
       if ((rc = launch_q4k_rows_segs(s, sg, d->width, xq, qkv))) return rc;
+    } else if (mixed_qkv && (d->neox || q8)) {
+      // a q8_0 cache or neox pairing: the same two launches, unrotated, for
+      // rope_store (a 4096x14336 layer at 8 tokens 177 us with a launch each
+      // for q, k and v on the int8 tiles, 139 with these)
+      if ((rc = launch_htile(s, MI_Q4_K, qk, qw + (int32_t)kvw, d->width, xq, hxn, tokens, qkv, qkv_stride,
+                             MI_EPI_NONE, nullptr)))
+        return rc;
+      if ((rc = launch_htile(s, MI_Q6_K, vs, (int32_t)kvw, d->width, xq, hxn, tokens, qkv + qw + kvw, qkv_stride,
+                             MI_EPI_NONE, nullptr)))
+        return rc;
     } else if (mixed_qkv) {
       // q|k with the rope and k's cache store on the Q4_K f16 tile, then v
       // on the Q6_K one, every row of which the same epilogue stores into
@@ -643,13 +652,13 @@ static int llama_layer(hipStream_t s, const mi_layer_desc* d, float* resid, uint
       }
     } else {
       if ((rc = launch_matvec(s, d->wq.kind, d->wq.data, d->wq.row_bytes, qw, d->width, xq, tokens, qkv,
-                              qkv_stride, MI_EPI_NONE, nullptr)))
+                              qkv_stride, MI_EPI_NONE, nullptr, hxn)))
         return rc;
       if ((rc = launch_matvec(s, d->wk.kind, d->wk.data, d->wk.row_bytes, (int32_t)kvw, d->width, xq, tokens,
-                              qkv + qw, qkv_stride, MI_EPI_NONE, nullptr)))
+                              qkv + qw, qkv_stride, MI_EPI_NONE, nullptr, hxn)))
         return rc;
       if ((rc = launch_matvec(s, d->wv.kind, d->wv.data, d->wv.row_bytes, (int32_t)kvw, d->width, xq, tokens,
-                              qkv + qw + kvw, qkv_stride, MI_EPI_NONE, nullptr)))
+                              qkv + qw + kvw, qkv_stride, MI_EPI_NONE, nullptr, hxn)))
         return rc;
     }
     // rotate q and k; k and v into the cache (f16, or q8_0 blocks encoded by

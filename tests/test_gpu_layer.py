@@ -720,3 +720,37 @@ def test_chained_layers_match_unchained(dims, tokens, family):
     xb, kb, vb = run(True)
     assert torch.equal(xa, xb)
     assert all(torch.equal(a, b) for a, b in zip(ka + va, kb + vb))
+
+
+@pytest.mark.parametrize("neox,form", [(0, "q8"), (1, "f16")])
+@pytest.mark.parametrize("width", [1024, 768])
+@pytest.mark.parametrize("tokens", [2, 8])
+def test_mixed_layer_unrotated(neox, form, width, tokens):
+    """Q4_K q and k with a Q6_K v where the rope is a launch of its own: on the
+    f16 tile at 1024 columns, the row kernels at 768; the batch gives each
+    sequence's own batch-1 layer within 1e-4 of the norm: sums are grouped
+    differently, and a key or value on the edge of its cache rounding may fall
+    to the other side (2^-11 or 1/254 of one of a head's 64 values)."""
+    from molla_amd import block, gpu
+    ctx = gpu.DeviceContext(0)
+    f = gpu.CACHE_Q8 if form == "q8" else gpu.CACHE_F16
+    spec = dict(spec_of(width, 1024, width // 64, width // 128, 64), neox=neox)
+    kinds = {n: oracle.Q4_K for n in ("wq", "wk", "wo", "gate", "up")}
+    kinds.update(wv=oracle.Q6_K, down=oracle.Q6_K)
+    bs, layer = device_layer_from(make_layer_weights(spec, 71, kinds), spec)
+    pos, row = 5, gpu.cache_row(f, bs.kv_width())
+    x = synth.normal(tokens * width, 72).cuda()
+
+    def run(xs, n):
+        k = torch.zeros(n * (pos + 1) * row, dtype=torch.float16, device="cuda")
+        v = torch.zeros_like(k)
+        posd = torch.full((n,), pos, dtype=torch.int32, device="cuda")
+        xs = xs.clone()
+        block.device_layer(ctx, layer, xs, k, v, (pos + 1) * row, posd, pos + 1, n, form=f)
+        ctx.synchronize()
+        return xs.cpu().double().reshape(n, width)
+
+    got = run(x, tokens)
+    want = torch.cat([run(x[t * width:(t + 1) * width], 1) for t in range(tokens)])
+    assert torch.isfinite(got).all()
+    assert (got - want).norm() <= 1e-4 * want.norm()
