@@ -6,7 +6,7 @@
     python -m molla_amd.trace_summary DB --first N  # each kernel's first N dispatches
     python -m molla_amd.trace_summary DB --steps N --cycle 'KERNEL=wo,down'
         # the same, the dispatches of KERNEL in each step labelled in turn
-    python -m molla_amd.trace_summary DB --calls prefill_x_kernel --per 23
+    python -m molla_amd.trace_summary DB --calls prefill_prep_kernel --per 23
         # calls that start at each dispatch of the named kernel, in runs of
         # 23 calls (one bench shape each): median duration per kernel
 
