@@ -20,10 +20,10 @@
 //   S^T = K Q^T, keys as rows (read straight from the cache) and queries as
 //   columns: a lane's 8 scores belong to its own query, the softmax takes two
 //   exchanges between lanes, and the weights are in place as the B operand of
-//   O^T = V^T P^T.  Queries enter as three halves (every bit of the f32), P as
-//   two after a lift by 2^14; values lie by rows in LDS and are read
-//   transposed (ds_read_b64_tr_b16).  Slot i of lane group g takes key
-//   4 g + i % 4 + 16 (i / 4), the order in which S^T leaves them.
+//   O^T = V^T P^T.  Queries enter as three halves, scaled to their largest value
+//   (as in attend_flash.hip), P as two after a lift by 2^14; values lie by rows
+//   in LDS and are read transposed (ds_read_b64_tr_b16).  Slot i of lane group
+//   g takes key 4 g + i % 4 + 16 (i / 4), the order in which S^T leaves them.
 //
 // q8_0: quants enter as exact halves; a key block's factor multiplies its part
 // of the score, a value block's the weights, held relative to the largest
@@ -174,198 +174,213 @@ __global__ __launch_bounds__(64 * kWaves, 2) void attend_decode_kernel(
       else vw[j] = *(const du4*)(vc + row_of(key0, cells, i / PIECES) + kvh * D + 8 * (i % PIECES));
     }
   };
-  int key0 = s0 * kStep + kRun * wave;
-  int cells = cells_of(key0);
-  load_k(key0, cells);
-  load_v(key0, cells);
-  int cells_next = cells_of(key0 + kStep);
-  __builtin_amdgcn_sched_barrier(0);
-
-  // the queries as B fragments: column lm (zero past the group)
-  const float c2 = fabsf(scale) * kLog2e;
-  dh8 qf[3][KS];
-  {
-    const float sgn = scale < 0.0f ? -1.0f : 1.0f;
-#pragma unroll
-    for (int ks = 0; ks < KS; ks++) {
-#pragma unroll
-      for (int u = 0; u < 8; u++) {
-        const float f = lm < group ? sgn * qraw[ks][u >> 2][u & 3] : 0.0f;
-        const _Float16 h1 = (_Float16)f;
-        const float r1 = f - (float)h1;  // exact
-        const _Float16 h2 = (_Float16)r1;
-        qf[0][ks][u] = h1;
-        qf[1][ks][u] = h2;
-        qf[2][ks][u] = (_Float16)(r1 - (float)h2);
-      }
-    }
-  }
-
-  typedef __attribute__((address_space(3))) char* lds_ptr;
-  const lds_ptr vl = (lds_ptr)&vs[wave][0];
-  float* fl = fac[wave];
-  // transposed reads: rows 4 lk + i16 / 4 (+ 16), dims 16 dt + 4 (i16 % 4): the
-  // slot is an exclusive or with bits a row's start leaves free
-  uint32_t vat[2];
-#pragma unroll
-  for (int v = 0; v < 2; v++) {
-    const int row = 4 * lk + (lm >> 2) + 16 * v;
-    vat[v] = 2 * row * D + 16 * (((lm & 3) >> 1) ^ swz<D>(row)) + 8 * (lm & 1);
-  }
   df4 o[NT];
 #pragma unroll
   for (int dt = 0; dt < NT; dt++) o[dt] = df4{0.0f, 0.0f, 0.0f, 0.0f};
   int xo[Q8 ? KS : 1];  // q8_0: the X that each 32-dim block of o is held at
 #pragma unroll
   for (int b = 0; b < (Q8 ? KS : 1); b++) xo[b] = -100;
-  float mc = -1e30f, l = 0.0f;  // the running maximum is of the scores, before c2
+  // this wave's maximum in base 2 and sum
+  float m2 = -INFINITY, l = 0.0f;
 
-  for (int sl = s0; sl < s1; sl++, key0 += kStep) {
-    if (key0 >= count) break;  // (uniform over the wave: no keys left for it)
-    df4 s[2];
-    if constexpr (Q8) {
-      // factors to LDS by (key | value, block, key), read back four keys a lane
+  int key0 = s0 * kStep + kRun * wave;
+  if (key0 < count) {  // (uniform over the wave; else it has no keys)
+    int cells = cells_of(key0);
+    load_k(key0, cells);
+    load_v(key0, cells);
+    int cells_next = cells_of(key0 + kStep);
+    __builtin_amdgcn_sched_barrier(0);
+
+    // the queries as B fragments: column lm (zero past the group), each scaled by
+    // a power of two that c2 takes back (as in attend_flash.hip)
+    float c2 = fabsf(scale) * kLog2e;
+    dh8 qf[3][KS];
+    {
+      float mx = 0.0f;
 #pragma unroll
-      for (int b = 0; b < KS; b++)
-        fl[(lane >> 5) * KS * kRun + b * kRun + (lane & 31)] = half_bits_to_float(b < 2 ? fw.x >> (16 * b) : fw.y >> (16 * (b - 2)));
-      asm volatile("" ::: "memory");
+      for (int ks = 0; ks < KS; ks++)
 #pragma unroll
-      for (int a = 0; a < 2; a++) {
-        s[a] = df4{0.0f, 0.0f, 0.0f, 0.0f};
+        for (int u = 0; u < 8; u++) mx = fmaxf(mx, fabsf(qraw[ks][u >> 2][u & 3]));
+      mx = across(mx, lanes::Max{});
+      const int e = mx > 0.0f ? max(__builtin_amdgcn_frexp_expf(mx) - 15, -126) : 0;
+      c2 = ldexpf(c2, e);
+      const float sc = lm < group ? ldexpf(scale < 0.0f ? -1.0f : 1.0f, -e) : 0.0f;
 #pragma unroll
-        for (int ks = 0; ks < KS; ks++) {
-          const dh8 k8 = int8_halves(kw[a][ks].x, kw[a][ks].y);
-          df4 c = {0.0f, 0.0f, 0.0f, 0.0f};
+      for (int ks = 0; ks < KS; ks++) {
 #pragma unroll
-          for (int h = 0; h < 3; h++) c = mfma16(k8, qf[h][ks], c);
-          const df4 f = *(const df4*)(fl + ks * kRun + 16 * a + 4 * lk);
-#pragma unroll
-          for (int i = 0; i < 4; i++) s[a][i] = fmaf(f[i], c[i], s[a][i]);
+        for (int u = 0; u < 8; u++) {
+          const float f = qraw[ks][u >> 2][u & 3] * sc;
+          const _Float16 h1 = (_Float16)f;
+          const float r1 = f - (float)h1;  // exact
+          const _Float16 h2 = (_Float16)r1;
+          qf[0][ks][u] = h1;
+          qf[1][ks][u] = h2;
+          qf[2][ks][u] = (_Float16)(r1 - (float)h2);
         }
       }
-    } else {
-#pragma unroll
-      for (int a = 0; a < 2; a++) {
-        s[a] = df4{0.0f, 0.0f, 0.0f, 0.0f};
-#pragma unroll
-        for (int ks = 0; ks < KS; ks++)
-#pragma unroll
-          for (int h = 0; h < 3; h++) s[a] = mfma16(__builtin_bit_cast(dh8, kw[a][ks]), qf[h][ks], s[a]);
-      }
     }
-    uint32_t held = 0xffffffffu;
-    if constexpr (PAGED) held = (uint32_t)__ballot(cells >= 0);
-    const int nk = min(kRun, count - key0);
-    if (nk < kRun) held &= (1u << nk) - 1u;
-    const bool more = key0 + kStep < count && sl + 1 < s1;  // uniform
-    if (more) load_k(key0 + kStep, cells_next);
 
-    // running maximum and weights of this lane's keys 16 a + 4 lk + i
-    const uint32_t mine = held >> (4 * lk);
-    float m = -INFINITY;
+    typedef __attribute__((address_space(3))) char* lds_ptr;
+    const lds_ptr vl = (lds_ptr)&vs[wave][0];
+    float* fl = fac[wave];
+    // transposed reads: rows 4 lk + i16 / 4 (+ 16), dims 16 dt + 4 (i16 % 4): the
+    // slot is an exclusive or with bits a row's start leaves free
+    uint32_t vat[2];
 #pragma unroll
-    for (int a = 0; a < 2; a++)
-#pragma unroll
-      for (int i = 0; i < 4; i++) {
-        s[a][i] = (mine >> (16 * a + i)) & 1 ? s[a][i] : -INFINITY;
-        m = fmaxf(m, s[a][i]);
-      }
-    m = across(m, lanes::Max{});
-    const float mn = fmaxf(mc, m);
-    if (__any(mn != mc)) {
-      const float f = __builtin_amdgcn_exp2f((mc - mn) * c2);
-      l *= f;
-#pragma unroll
-      for (int dt = 0; dt < NT; dt++) o[dt] *= f;
-      mc = mn;
+    for (int v = 0; v < 2; v++) {
+      const int row = 4 * lk + (lm >> 2) + 16 * v;
+      vat[v] = 2 * row * D + 16 * (((lm & 3) >> 1) ^ swz<D>(row)) + 8 * (lm & 1);
     }
-    float p[8];
-#pragma unroll
-    for (int a = 0; a < 2; a++)
-#pragma unroll
-      for (int i = 0; i < 4; i++) {
-        const float e = __builtin_amdgcn_exp2f(fmaf(s[a][i] - mc, c2, kLift));  // (as in attend_flash.hip)
-        p[4 * a + i] = (mine >> (16 * a + i)) & 1 ? e : 0.0f;
-        l += p[4 * a + i];
-      }
+    float mc = -1e30f;  // the running maximum, of the scores before c2
 
-    // the values to this wave's LDS rows
-#pragma unroll
-    for (int j = 0; j < VW; j++) {
-      const int i = lane + 64 * j;
+    for (int sl = s0; sl < s1; sl++, key0 += kStep) {
+      if (key0 >= count) break;  // (uniform over the wave: no keys left for it)
+      df4 s[2];
       if constexpr (Q8) {
-        const int row = i / (D / 16), pc = 2 * (i % (D / 16));
-        *(__attribute__((address_space(3))) dh8*)(vl + 2 * row * D + 16 * (pc ^ swz<D>(row))) = int8_halves(vw[j].x, vw[j].y);
-        *(__attribute__((address_space(3))) dh8*)(vl + 2 * row * D + 16 * ((pc + 1) ^ swz<D>(row))) = int8_halves(vw[j].z, vw[j].w);
+        // factors to LDS by (key | value, block, key), read back four keys a lane
+#pragma unroll
+        for (int b = 0; b < KS; b++)
+          fl[(lane >> 5) * KS * kRun + b * kRun + (lane & 31)] = half_bits_to_float(b < 2 ? fw.x >> (16 * b) : fw.y >> (16 * (b - 2)));
+        asm volatile("" ::: "memory");
+#pragma unroll
+        for (int a = 0; a < 2; a++) {
+          s[a] = df4{0.0f, 0.0f, 0.0f, 0.0f};
+#pragma unroll
+          for (int ks = 0; ks < KS; ks++) {
+            const dh8 k8 = int8_halves(kw[a][ks].x, kw[a][ks].y);
+            df4 c = {0.0f, 0.0f, 0.0f, 0.0f};
+#pragma unroll
+            for (int h = 0; h < 3; h++) c = mfma16(k8, qf[h][ks], c);
+            const df4 f = *(const df4*)(fl + ks * kRun + 16 * a + 4 * lk);
+#pragma unroll
+            for (int i = 0; i < 4; i++) s[a][i] = fmaf(f[i], c[i], s[a][i]);
+          }
+        }
       } else {
-        const int row = i / PIECES, pc = i % PIECES;
-        *(__attribute__((address_space(3))) du4*)(vl + 2 * row * D + 16 * (pc ^ swz<D>(row))) = vw[j];
-      }
-    }
-    df4 fv[Q8 ? KS : 1][2];
-    if constexpr (Q8) {
 #pragma unroll
-      for (int b = 0; b < KS; b++)
+        for (int a = 0; a < 2; a++) {
+          s[a] = df4{0.0f, 0.0f, 0.0f, 0.0f};
 #pragma unroll
-        for (int a = 0; a < 2; a++) fv[b][a] = *(const df4*)(fl + KS * kRun + b * kRun + 16 * a + 4 * lk);
-    }
-    asm volatile("" ::: "memory");  // (a wave's LDS operations complete in order)
-    if (more) load_v(key0 + kStep, cells_next);
-    cells = cells_next;
-    cells_next = cells_of(key0 + 2 * kStep);
-
-    dh8 ph, pl;
-    if constexpr (!Q8) {
+          for (int ks = 0; ks < KS; ks++)
 #pragma unroll
-      for (int i = 0; i < 8; i++) {
-        ph[i] = (_Float16)p[i];
-        pl[i] = (_Float16)(p[i] - (float)ph[i]);
-      }
-    }
-#pragma unroll
-    for (int dt = 0; dt < NT; dt++) {
-      if constexpr (Q8) {
-        if (dt % 2 == 0) {
-          const int b = dt / 2;
-          float fm = 0.0f;
-#pragma unroll
-          for (int i = 0; i < 8; i++) fm = fmaxf(fm, fabsf(fv[b][i >> 2][i & 3]));
-          fm = across(fm, lanes::Max{});
-          const int x = __builtin_amdgcn_readfirstlane(fm > 0.0f ? max(xo[b], __builtin_amdgcn_frexp_expf(fm)) : xo[b]);
-          if (x != xo[b]) {
-            const float f = ldexpf(1.0f, xo[b] - x);
-            o[dt] *= f;
-            o[dt + 1] *= f;
-            xo[b] = x;
-          }
-          const float unit = ldexpf(1.0f, -x);
-#pragma unroll
-          for (int i = 0; i < 8; i++) {
-            // rounded once: contracted into the two conversions, the halves
-            // came from two roundings of the product, a last bit of hi apart
-            float w = p[i] * (fv[b][i >> 2][i & 3] * unit);
-            asm("" : "+v"(w));
-            ph[i] = (_Float16)w;
-            pl[i] = (_Float16)(w - (float)ph[i]);
-          }
+            for (int h = 0; h < 3; h++) s[a] = mfma16(__builtin_bit_cast(dh8, kw[a][ks]), qf[h][ks], s[a]);
         }
       }
-      ds8 a;
+      uint32_t held = 0xffffffffu;
+      if constexpr (PAGED) held = (uint32_t)__ballot(cells >= 0);
+      const int nk = min(kRun, count - key0);
+      if (nk < kRun) held &= (1u << nk) - 1u;
+      const bool more = key0 + kStep < count && sl + 1 < s1;  // uniform
+      if (more) load_k(key0 + kStep, cells_next);
+
+      // running maximum and weights of this lane's keys 16 a + 4 lk + i
+      const uint32_t mine = held >> (4 * lk);
+      float m = -INFINITY;
 #pragma unroll
-      for (int v = 0; v < 2; v++) {
-        const ds4 x = __builtin_amdgcn_ds_read_tr16_b64_v4i16(
-            (__attribute__((address_space(3))) ds4*)(vl + (vat[v] ^ (32 * dt))));
+      for (int a = 0; a < 2; a++)
 #pragma unroll
-        for (int e = 0; e < 4; e++) a[4 * v + e] = x[e];
+        for (int i = 0; i < 4; i++) {
+          s[a][i] = (mine >> (16 * a + i)) & 1 ? s[a][i] : -INFINITY;
+          m = fmaxf(m, s[a][i]);
+        }
+      m = across(m, lanes::Max{});
+      const float mn = fmaxf(mc, m);
+      if (__any(mn != mc)) {
+        const float f = __builtin_amdgcn_exp2f((mc - mn) * c2);
+        l *= f;
+#pragma unroll
+        for (int dt = 0; dt < NT; dt++) o[dt] *= f;
+        mc = mn;
       }
-      o[dt] = mfma16(__builtin_bit_cast(dh8, a), ph, o[dt]);
-      o[dt] = mfma16(__builtin_bit_cast(dh8, a), pl, o[dt]);
+      float p[8];
+#pragma unroll
+      for (int a = 0; a < 2; a++)
+#pragma unroll
+        for (int i = 0; i < 4; i++) {
+          const float e = __builtin_amdgcn_exp2f(fmaf(s[a][i] - mc, c2, kLift));  // (as in attend_flash.hip)
+          p[4 * a + i] = (mine >> (16 * a + i)) & 1 ? e : 0.0f;
+          l += p[4 * a + i];
+        }
+
+      // the values to this wave's LDS rows
+#pragma unroll
+      for (int j = 0; j < VW; j++) {
+        const int i = lane + 64 * j;
+        if constexpr (Q8) {
+          const int row = i / (D / 16), pc = 2 * (i % (D / 16));
+          *(__attribute__((address_space(3))) dh8*)(vl + 2 * row * D + 16 * (pc ^ swz<D>(row))) = int8_halves(vw[j].x, vw[j].y);
+          *(__attribute__((address_space(3))) dh8*)(vl + 2 * row * D + 16 * ((pc + 1) ^ swz<D>(row))) = int8_halves(vw[j].z, vw[j].w);
+        } else {
+          const int row = i / PIECES, pc = i % PIECES;
+          *(__attribute__((address_space(3))) du4*)(vl + 2 * row * D + 16 * (pc ^ swz<D>(row))) = vw[j];
+        }
+      }
+      df4 fv[Q8 ? KS : 1][2];
+      if constexpr (Q8) {
+#pragma unroll
+        for (int b = 0; b < KS; b++)
+#pragma unroll
+          for (int a = 0; a < 2; a++) fv[b][a] = *(const df4*)(fl + KS * kRun + b * kRun + 16 * a + 4 * lk);
+      }
+      asm volatile("" ::: "memory");  // (a wave's LDS operations complete in order)
+      if (more) load_v(key0 + kStep, cells_next);
+      cells = cells_next;
+      cells_next = cells_of(key0 + 2 * kStep);
+
+      dh8 ph, pl;
+      if constexpr (!Q8) {
+#pragma unroll
+        for (int i = 0; i < 8; i++) {
+          ph[i] = (_Float16)p[i];
+          pl[i] = (_Float16)(p[i] - (float)ph[i]);
+        }
+      }
+#pragma unroll
+      for (int dt = 0; dt < NT; dt++) {
+        if constexpr (Q8) {
+          if (dt % 2 == 0) {
+            const int b = dt / 2;
+            float fm = 0.0f;
+#pragma unroll
+            for (int i = 0; i < 8; i++) fm = fmaxf(fm, fabsf(fv[b][i >> 2][i & 3]));
+            fm = across(fm, lanes::Max{});
+            const int x = __builtin_amdgcn_readfirstlane(fm > 0.0f ? max(xo[b], __builtin_amdgcn_frexp_expf(fm)) : xo[b]);
+            if (x != xo[b]) {
+              const float f = ldexpf(1.0f, xo[b] - x);
+              o[dt] *= f;
+              o[dt + 1] *= f;
+              xo[b] = x;
+            }
+            const float unit = ldexpf(1.0f, -x);
+#pragma unroll
+            for (int i = 0; i < 8; i++) {
+              // rounded once: contracted into the two conversions, the halves
+              // came from two roundings of the product, a last bit of hi apart
+              float w = p[i] * (fv[b][i >> 2][i & 3] * unit);
+              asm("" : "+v"(w));
+              ph[i] = (_Float16)w;
+              pl[i] = (_Float16)(w - (float)ph[i]);
+            }
+          }
+        }
+        ds8 a;
+#pragma unroll
+        for (int v = 0; v < 2; v++) {
+          const ds4 x = __builtin_amdgcn_ds_read_tr16_b64_v4i16(
+              (__attribute__((address_space(3))) ds4*)(vl + (vat[v] ^ (32 * dt))));
+#pragma unroll
+          for (int e = 0; e < 4; e++) a[4 * v + e] = x[e];
+        }
+        o[dt] = mfma16(__builtin_bit_cast(dh8, a), ph, o[dt]);
+        o[dt] = mfma16(__builtin_bit_cast(dh8, a), pl, o[dt]);
+      }
+      asm volatile("" ::: "memory");  // the reads above stay ahead of the next run's stores
     }
-    asm volatile("" ::: "memory");  // the reads above stay ahead of the next run's stores
+    l = across(l, lanes::Add{});
+    if (l != 0.0f) m2 = mc * c2;  // (no key held: no part in the fold)
   }
 
   // fold the waves: their sums (in place of the values) and (maximum, sum)
-  l = across(l, lanes::Add{});
   float* wo = (float*)&vs[0][0];  // [wave][group][D]
   __syncthreads();
   if (lm < group) {
@@ -375,16 +390,16 @@ __global__ __launch_bounds__(64 * kWaves, 2) void attend_decode_kernel(
       *(df4*)(wo + (wave * group + lm) * D + 16 * dt + 4 * lk) = o[dt];
     }
     if (lk == 0) {
-      wml[wave][0][lm] = mc * c2;
+      wml[wave][0][lm] = m2;
       wml[wave][1][lm] = l;
     }
   }
   __syncthreads();
   for (int i = tid; i < group * D; i += 64 * kWaves) {
     const int g = i / D, d = i - g * D;
-    float m = wml[0][0][g];
+    float m = -3e38f;
 #pragma unroll
-    for (int w = 1; w < kWaves; w++) m = fmaxf(m, wml[w][0][g]);
+    for (int w = 0; w < kWaves; w++) m = fmaxf(m, wml[w][0][g]);
     float v = 0.0f, sum = 0.0f;
 #pragma unroll
     for (int w = 0; w < kWaves; w++) {

@@ -14,8 +14,10 @@
 //   S^T = K Q^T, keys as rows and queries as columns: a lane's 32 scores of a
 //   slice all belong to its own query, so the softmax is in the lane but for
 //   one exchange of the two half waves, and the weights are in place as the B
-//   operand of the next product.  Queries enter as three halves (every bit of
-//   the f32 query: two left 1e-4 of the output at scores of a few hundred).
+//   operand of the next product.  Queries enter as three halves, each query
+//   scaled by a power of two so that its largest value is in [2^14, 2^15): any
+//   f32 query, to 2^-39 of its largest value (every bit of values down to 2^-15
+//   of it; two halves left 1e-4 of the output at scores of a few hundred).
 //   O^T = V^T P^T: values lie by rows in LDS and are read transposed
 //   (ds_read_b64_tr_b16); P is lifted by 2^14 and split into two halves (see
 //   kLift).  MFMA step u of a 32-key tile takes keys 8 (i / 4) + 4 h + i % 4
@@ -133,18 +135,33 @@ __global__ __launch_bounds__(256, 2) void attend_flash_kernel(
   const int slices = (count + kSlice - 1) / kSlice, per = (slices + splits - 1) / splits;
   const int s0 = split * per, s1 = min(s0 + per, slices);
 
-  // scores are taken against |scale| log2(e), the query carrying its sign
-  const float c2 = fabsf(scale) * kLog2e;
+  // The query, scaled by the power of two that brings its largest value to
+  // [2^14, 2^15) and split into three halves; scores are taken against |scale|
+  // log2(e), which takes the power back, the query carrying scale's sign.
+  float c2 = fabsf(scale) * kLog2e;
   fh8 qf[3][D / 16];
   {
-    const float sgn = scale < 0.0f ? -1.0f : 1.0f;
     const float* qr = q + (int64_t)min(t, tokens - 1) * q_stride + (int64_t)head * D + 8 * h;
+    ff4 raw[D / 16][2];
+    float mx = 0.0f;
 #pragma unroll
     for (int st = 0; st < D / 16; st++) {
-      const ff4 a = *(const ff4*)(qr + 16 * st), b = *(const ff4*)(qr + 16 * st + 4);
+      raw[st][0] = *(const ff4*)(qr + 16 * st);
+      raw[st][1] = *(const ff4*)(qr + 16 * st + 4);
+    }
+#pragma unroll
+    for (int st = 0; st < D / 16; st++)
+#pragma unroll
+      for (int u = 0; u < 8; u++) mx = fmaxf(mx, fabsf(raw[st][u >> 2][u & 3]));
+    mx = other_max(mx);
+    const int e = mx > 0.0f ? max(__builtin_amdgcn_frexp_expf(mx) - 15, -126) : 0;
+    c2 = ldexpf(c2, e);
+    const float sc = ldexpf(scale < 0.0f ? -1.0f : 1.0f, -e);
+#pragma unroll
+    for (int st = 0; st < D / 16; st++) {
 #pragma unroll
       for (int u = 0; u < 8; u++) {
-        const float f = sgn * (u < 4 ? a[u & 3] : b[u & 3]);
+        const float f = sc * raw[st][u >> 2][u & 3];
         const _Float16 h1 = (_Float16)f;
         const float r1 = f - (float)h1;  // exact
         const _Float16 h2 = (_Float16)r1;

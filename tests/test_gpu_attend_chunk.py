@@ -91,3 +91,36 @@ def test_chunk_attention_edges(form, dims, first, tokens, paged):
         bound = layer_gate(spec, host, xr, kr, vr, slot)
         oracle.layer_step(L, xr, kr, vr, slot, p, f16_store=not q8, q8_store=q8, threads=8)
         assert_layer_close(xd.cpu().numpy().reshape(tokens, -1)[i], xr, bound, f"token {i}:")
+
+
+@pytest.mark.parametrize("form", ["f16", "q8"])
+@pytest.mark.parametrize("dims", [(512, 256, 8, 2, 64), (1024, 256, 8, 1, 128)])
+@pytest.mark.parametrize("power", [-40, -12, 20, 60])
+def test_chunk_query_of_any_size(form, dims, power):
+    """Queries times 2^power (the gain of the per-head query norm) and the
+    attention scale times 2^-power are the same scores: the layer is the same
+    to the bit (a half alone would overflow from 2^16 on, and lose its low bits
+    below 1/2)."""
+    from molla_amd import block, gpu
+    ctx = gpu.DeviceContext(0)
+    f = gpu.CACHE_Q8 if form == "q8" else gpu.CACHE_F16
+    spec = spec_of(*dims)
+    first, tokens = 70, 40
+    bs, layer = device_layer_from(make_layer_weights(spec, 27), spec)
+    kvw, hd, count = bs.kv_width(), dims[4], first + tokens
+    k, v = (synth.normal(count * kvw, 94 + i) for i in (0, 1))
+    if form == "q8":
+        from tests.test_gpu_kernels import q8_rows
+        k, v = (torch.from_numpy(q8_rows(c.numpy(), kvw).view(np.int16).copy()).view(torch.float16) for c in (k, v))
+    x = synth.normal(tokens * bs.width, 96).cuda()
+    posd = torch.arange(first, count, dtype=torch.int32, device="cuda")
+    ones = torch.ones(hd, device="cuda")
+    outs = []
+    for p in (0, power):
+        l = block.DeviceLayer(bs, layer.attn_norm, layer.ffn_norm, layer.weights, layer.rope_steps,
+                              extras={"q_norm": ones * 2.0 ** p, "k_norm": ones})
+        l.desc.attn_scale = 2.0 ** (-3 - p)
+        xd, kd, vd = x.clone(), k.half().cuda(), v.half().cuda()
+        block.device_layer(ctx, l, xd, kd, vd, 0, posd, count, tokens, form=f)
+        outs.append(xd.cpu())
+    assert torch.isfinite(outs[0]).all() and torch.equal(outs[0], outs[1])

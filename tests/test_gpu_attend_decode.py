@@ -88,3 +88,49 @@ def test_context_longer_than_the_position(form, tokens):
         outs.append(xd.cpu().double())
     assert torch.isfinite(outs[1]).all()
     assert (outs[0] - outs[1]).norm() <= 1e-5 * outs[0].norm()
+
+
+@pytest.mark.parametrize("form", ["f16", "q8"])
+@pytest.mark.parametrize("heads,kv,hd", [(8, 2, 128), (8, 1, 64)])
+@pytest.mark.parametrize("power", [-90, -40, -12, 4, 20, 100])
+def test_query_of_any_size(form, heads, kv, hd, power):
+    """A query times 2^power and the scale times 2^-power are the same scores:
+    the result is the same to the bit, whatever the query's size (a half alone
+    would overflow from 2^16 on, and lose its low bits below 1/2)."""
+    from molla_amd import gpu
+    ctx = gpu.DeviceContext(0)
+    count = 300
+    (kd, vd), _ = caches(form, count, kv * hd, 70)
+    q = synth.normal(heads * hd, 72).cuda()
+    f = gpu.CACHE_Q8 if form == "q8" else gpu.CACHE_F16
+    outs = []
+    for p in (0, power):
+        out = torch.zeros(heads * hd, device="cuda")
+        # (no query value and neither scale leaves the normal floats)
+        gpu.device_attend(ctx, q * 2.0 ** p, kd, vd, heads, kv, hd, 2.0 ** (-3 - p), count, out, f)
+        outs.append(out.cpu())
+    assert torch.isfinite(outs[0]).all() and torch.equal(outs[0], outs[1])
+
+
+@pytest.mark.parametrize("form", ["f16", "q8"])
+@pytest.mark.parametrize("size,keys", [(1e6, 1.0), (1e-6, 1e4)])
+def test_large_and_small_queries(form, size, keys):
+    """The same against the oracle, with the keys as they are in a cache of
+    large ones: scores of a few units."""
+    from molla_amd import gpu
+    from tests.test_gpu_kernels import q8_decode, q8_rows
+    ctx = gpu.DeviceContext(0)
+    heads, kv, hd, count = 16, 2, 128, 400
+    dev, host = [], []
+    for i, m in enumerate((keys, 1.0)):
+        raw = synth.normal(count * kv * hd, 80 + i).numpy() * np.float32(m)
+        h = q8_rows(raw, kv * hd) if form == "q8" else raw.astype(np.float16).view(np.uint16)
+        dev.append(torch.from_numpy(h.view(np.int16).copy()).view(torch.float16).cuda())
+        host.append(q8_decode(h, kv * hd, count).reshape(-1) if form == "q8" else h.view(np.float16).astype(np.float32))
+    q = synth.normal(heads * hd, 82).numpy() * np.float32(size)
+    scale = float(np.float32(1 / np.sqrt(hd) / size / keys))
+    out = torch.zeros(heads * hd, device="cuda")
+    gpu.device_attend(ctx, torch.from_numpy(q).cuda(), dev[0], dev[1], heads, kv, hd, scale, count, out,
+                      gpu.CACHE_Q8 if form == "q8" else gpu.CACHE_F16)
+    want = oracle.attend(heads, kv, hd, scale, q, host[0], host[1], count)
+    assert np.abs(out.cpu().numpy() - want).max() <= 1e-5 * np.abs(want).max()
