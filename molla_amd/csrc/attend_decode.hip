@@ -26,8 +26,10 @@
 //   g takes key 4 g + i % 4 + 16 (i / 4), the order in which S^T leaves them.
 //
 // q8_0: quants enter as exact halves; a key block's factor multiplies its part
-// of the score, a value block's the weights, held relative to the largest
-// factor so far of that block of 32 dims (2^-X) so that no half is subnormal.
+// of the score, a value block's the weights.  The products enter as two halves,
+// scaled by 2^(15 - X) with X the exponent of the column's largest one since its
+// maximum last rose: to 2^-39 of that, whatever the factors' range.  A key that
+// is not there has a factor of 0.
 //
 // MFMA fragments (16x16x32): lane l holds row / column l % 16 and values
 // 8 (l / 16) .. +8 of the 32; result element i of lane l is row 4 (l / 16) +
@@ -177,7 +179,7 @@ __global__ __launch_bounds__(64 * kWaves, 2) void attend_decode_kernel(
   df4 o[NT];
 #pragma unroll
   for (int dt = 0; dt < NT; dt++) o[dt] = df4{0.0f, 0.0f, 0.0f, 0.0f};
-  int xo[Q8 ? KS : 1];  // q8_0: the X that each 32-dim block of o is held at
+  int xo[Q8 ? KS : 1];  // q8_0: the X that this column's 32-dim blocks of o are held at
 #pragma unroll
   for (int b = 0; b < (Q8 ? KS : 1); b++) xo[b] = -100;
   // this wave's maximum in base 2 and sum
@@ -235,9 +237,15 @@ __global__ __launch_bounds__(64 * kWaves, 2) void attend_decode_kernel(
 
     for (int sl = s0; sl < s1; sl++, key0 += kStep) {
       if (key0 >= count) break;  // (uniform over the wave: no keys left for it)
+      uint32_t held = 0xffffffffu;
+      if constexpr (PAGED) held = (uint32_t)__ballot(cells >= 0);
+      const int nk = min(kRun, count - key0);
+      if (nk < kRun) held &= (1u << nk) - 1u;
       df4 s[2];
       if constexpr (Q8) {
-        // factors to LDS by (key | value, block, key), read back four keys a lane
+        // factors to LDS by (key | value, block, key), read back four keys a
+        // lane; zero for a key past the end or not held, whose row is another's
+        if (!((held >> (lane & 31)) & 1)) fw = du2{0, 0};
 #pragma unroll
         for (int b = 0; b < KS; b++)
           fl[(lane >> 5) * KS * kRun + b * kRun + (lane & 31)] = half_bits_to_float(b < 2 ? fw.x >> (16 * b) : fw.y >> (16 * (b - 2)));
@@ -266,10 +274,6 @@ __global__ __launch_bounds__(64 * kWaves, 2) void attend_decode_kernel(
             for (int h = 0; h < 3; h++) s[a] = mfma16(__builtin_bit_cast(dh8, kw[a][ks]), qf[h][ks], s[a]);
         }
       }
-      uint32_t held = 0xffffffffu;
-      if constexpr (PAGED) held = (uint32_t)__ballot(cells >= 0);
-      const int nk = min(kRun, count - key0);
-      if (nk < kRun) held &= (1u << nk) - 1u;
       const bool more = key0 + kStep < count && sl + 1 < s1;  // uniform
       if (more) load_k(key0 + kStep, cells_next);
 
@@ -285,7 +289,8 @@ __global__ __launch_bounds__(64 * kWaves, 2) void attend_decode_kernel(
         }
       m = across(m, lanes::Max{});
       const float mn = fmaxf(mc, m);
-      if (__any(mn != mc)) {
+      const bool rose = mn != mc;
+      if (__any(rose)) {
         const float f = __builtin_amdgcn_exp2f((mc - mn) * c2);
         l *= f;
 #pragma unroll
@@ -340,26 +345,33 @@ __global__ __launch_bounds__(64 * kWaves, 2) void attend_decode_kernel(
         if constexpr (Q8) {
           if (dt % 2 == 0) {
             const int b = dt / 2;
-            float fm = 0.0f;
+            float w[8], wm = 0.0f;
 #pragma unroll
-            for (int i = 0; i < 8; i++) fm = fmaxf(fm, fabsf(fv[b][i >> 2][i & 3]));
-            fm = across(fm, lanes::Max{});
-            const int x = __builtin_amdgcn_readfirstlane(fm > 0.0f ? max(xo[b], __builtin_amdgcn_frexp_expf(fm)) : xo[b]);
-            if (x != xo[b]) {
+            for (int i = 0; i < 8; i++) {
+              w[i] = p[i] * fv[b][i >> 2][i & 3];
+              wm = fmaxf(wm, fabsf(w[i]));
+            }
+            wm = across(wm, lanes::Max{});
+            // (an infinite factor: the finite products are below 2^31)
+            const int xw = wm < INFINITY ? __builtin_amdgcn_frexp_expf(wm) : 31;
+            const int x = wm > 0.0f ? max(max(xw, rose ? xo[b] - 60 : xo[b]), -100) : xo[b];
+            if (__any(x != xo[b])) {
               const float f = ldexpf(1.0f, xo[b] - x);
               o[dt] *= f;
               o[dt + 1] *= f;
               xo[b] = x;
             }
-            const float unit = ldexpf(1.0f, -x);
+            const float unit = ldexpf(1.0f, 15 - x);
 #pragma unroll
             for (int i = 0; i < 8; i++) {
-              // rounded once: contracted into the two conversions, the halves
-              // came from two roundings of the product, a last bit of hi apart
-              float w = p[i] * (fv[b][i >> 2][i & 3] * unit);
-              asm("" : "+v"(w));
-              ph[i] = (_Float16)w;
-              pl[i] = (_Float16)(w - (float)ph[i]);
+              const float v = w[i] * unit;
+              ph[i] = (_Float16)v;
+              pl[i] = (_Float16)(v - (float)ph[i]);
+            }
+            if (__builtin_expect(__any(!(wm < INFINITY)), 0)) {
+#pragma unroll
+              for (int i = 0; i < 8; i++)
+                if (!(fabsf(w[i]) < INFINITY)) pl[i] = 0;
             }
           }
         }
@@ -386,7 +398,7 @@ __global__ __launch_bounds__(64 * kWaves, 2) void attend_decode_kernel(
   if (lm < group) {
 #pragma unroll
     for (int dt = 0; dt < NT; dt++) {
-      if constexpr (Q8) o[dt] *= ldexpf(1.0f, xo[dt / 2]);
+      if constexpr (Q8) o[dt] *= ldexpf(1.0f, xo[dt / 2] - 15);
       *(df4*)(wo + (wave * group + lm) * D + 16 * dt + 4 * lk) = o[dt];
     }
     if (lk == 0) {

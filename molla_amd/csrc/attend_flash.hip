@@ -26,7 +26,11 @@
 // q8_0: keys enter as their integers (exact halves) and each 32-value
 // block's factor multiplies that block's part of the score; values enter as
 // value * 2^(8 - X) in two halves (7 + 11 bits: exact), X the largest factor's
-// exponent so far in that 32-value block, so that neither half is subnormal.
+// exponent so far in that 32-value block.  A key whose factor is below
+// 2^(X - 22) (its low half would be subnormal) or not finite is left out of the
+// product (its values enter as zeros) and added in float32 at the end, to the
+// rows that it is live for: a later token's factor changes nothing of an earlier
+// one's result.
 //
 // MFMA fragments (32x32x16): lane l holds row / column l % 32 and values
 // 8 (l / 32) .. +8 of the 16; result element j of lane l is row 8 (j / 4) +
@@ -118,6 +122,7 @@ __global__ __launch_bounds__(256, 2) void attend_flash_kernel(
   __shared__ __align__(16) _Float16 vs[VB * VH][kSlice * D];
   __shared__ __align__(16) float kf[Q8 ? 2 : 1][Q8 ? NT : 1][kSlice];  // q8_0 key factors
   __shared__ int vexp[Q8 ? 4 : 1];                                     // X of each wave's dims
+  __shared__ int left_out;                                             // q8_0: some key's values were
   __shared__ int cmax[4];
   const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
   const int n = lane & 31, h = lane >> 5;
@@ -130,46 +135,23 @@ __global__ __launch_bounds__(256, 2) void attend_flash_kernel(
   const int wave_max = lanes::reduce<64>(cnt, IMax{});
   const int wave_min = -lanes::reduce<64>(live_row ? -cnt : -0x7fffffff, IMax{});
   if (lane == 0) cmax[wave] = wave_max;
+  if (Q8 && tid == 0) left_out = 0;
   __syncthreads();
   const int count = __builtin_amdgcn_readfirstlane(max(max(cmax[0], cmax[1]), max(cmax[2], cmax[3])));
   const int slices = (count + kSlice - 1) / kSlice, per = (slices + splits - 1) / splits;
   const int s0 = split * per, s1 = min(s0 + per, slices);
 
-  // The query, scaled by the power of two that brings its largest value to
-  // [2^14, 2^15) and split into three halves; scores are taken against |scale|
-  // log2(e), which takes the power back, the query carrying scale's sign.
-  float c2 = fabsf(scale) * kLog2e;
-  fh8 qf[3][D / 16];
-  {
-    const float* qr = q + (int64_t)min(t, tokens - 1) * q_stride + (int64_t)head * D + 8 * h;
-    ff4 raw[D / 16][2];
-    float mx = 0.0f;
+  if (s0 >= s1) {  // (uniform; only with several splits) no keys: no part in the fold
+    if (live_row && h == 0) *(float2*)(part_ml + (((int64_t)t * heads + head) * splits + split) * 2) = make_float2(0.0f, 0.0f);
+    return;
+  }
+
+  const float* qr = q + (int64_t)min(t, tokens - 1) * q_stride + (int64_t)head * D + 8 * h;
+  ff4 qraw[D / 16][2];
 #pragma unroll
-    for (int st = 0; st < D / 16; st++) {
-      raw[st][0] = *(const ff4*)(qr + 16 * st);
-      raw[st][1] = *(const ff4*)(qr + 16 * st + 4);
-    }
-#pragma unroll
-    for (int st = 0; st < D / 16; st++)
-#pragma unroll
-      for (int u = 0; u < 8; u++) mx = fmaxf(mx, fabsf(raw[st][u >> 2][u & 3]));
-    mx = other_max(mx);
-    const int e = mx > 0.0f ? max(__builtin_amdgcn_frexp_expf(mx) - 15, -126) : 0;
-    c2 = ldexpf(c2, e);
-    const float sc = ldexpf(scale < 0.0f ? -1.0f : 1.0f, -e);
-#pragma unroll
-    for (int st = 0; st < D / 16; st++) {
-#pragma unroll
-      for (int u = 0; u < 8; u++) {
-        const float f = sc * raw[st][u >> 2][u & 3];
-        const _Float16 h1 = (_Float16)f;
-        const float r1 = f - (float)h1;  // exact
-        const _Float16 h2 = (_Float16)r1;
-        qf[0][st][u] = h1;
-        qf[1][st][u] = h2;
-        qf[2][st][u] = (_Float16)(r1 - (float)h2);
-      }
-    }
+  for (int st = 0; st < D / 16; st++) {
+    qraw[st][0] = *(const ff4*)(qr + 16 * st);
+    qraw[st][1] = *(const ff4*)(qr + 16 * st + 4);
   }
 
   // Staging.  f16: a thread copies pieces tid + 256 j of the slice's rows.
@@ -177,24 +159,28 @@ __global__ __launch_bounds__(256, 2) void attend_flash_kernel(
   // one 32-value block).  Keys past the end repeat the last one (masked).
   constexpr int PER = Q8 ? D / 64 : kSlice * PIECES / 256;  // 16-byte words of K (and of V)
   fu4 kr[PER], vr[PER];
-  float kfr = 0.0f, vfr = 0.0f;
+  uint16_t kfr = 0, vfr = 0;  // the factor's bits (converted when stored: a use here would wait for the load)
+  uint64_t dead = 0;  // q8_0: the loaded slice's keys that no row reaches
   const int kvw = kv_heads * D;
   auto cell_of = [&](int sl, int key) __attribute__((always_inline)) {
     const int j = min(sl * kSlice + key, count - 1);
-    return (int64_t)(PAGED ? max(kv_index[j], 0) : j) * row_halves;
+    return PAGED ? kv_index[j] : j;  // (negative: not held)
   };
-  auto load = [&](const __half* __restrict__ c, int sl, fu4 (&w)[PER], float& f) __attribute__((always_inline)) {
+  auto row_of = [&](int cell) __attribute__((always_inline)) { return (int64_t)max(cell, 0) * row_halves; };
+  auto load = [&](const __half* __restrict__ c, int sl, fu4 (&w)[PER], uint16_t& f) __attribute__((always_inline)) {
     if constexpr (Q8) {
-      const __half* rowp = c + cell_of(sl, lane);
+      const int cell = cell_of(sl, lane);
+      const __half* rowp = c + row_of(cell);
       const int8_t* b = (const int8_t*)rowp + kvh * D + wave * (D / 4);
 #pragma unroll
       for (int j = 0; j < PER; j++) w[j] = *(const fu4*)(b + 16 * j);
-      f = __half2float(rowp[(kvw >> 1) + ((kvh * D + wave * (D / 4)) >> 5)]);
+      f = ((const uint16_t*)rowp)[(kvw >> 1) + ((kvh * D + wave * (D / 4)) >> 5)];
+      dead = __ballot(sl * kSlice + lane >= count || (PAGED && cell < 0));
     } else {
 #pragma unroll
       for (int j = 0; j < PER; j++) {
         const int i = tid + 256 * j;
-        w[j] = *(const fu4*)(c + cell_of(sl, i / PIECES) + kvh * D + 8 * (i % PIECES));
+        w[j] = *(const fu4*)(c + row_of(cell_of(sl, i / PIECES)) + kvh * D + 8 * (i % PIECES));
       }
     }
   };
@@ -217,7 +203,7 @@ __global__ __launch_bounds__(256, 2) void attend_flash_kernel(
         *(fh8*)(ks[buf] + lane * D + 8 * ((pc + 1) ^ key_swz<D>(lane))) = a[1];
       }
       // (at D = 64 two waves share a block and write the same factors)
-      kf[buf][wave * (D / 4) / 32][lane] = kfr;
+      kf[buf][wave * (D / 4) / 32][lane] = half_bits_to_float(kfr);
     } else {
 #pragma unroll
       for (int j = 0; j < PER; j++) {
@@ -226,14 +212,24 @@ __global__ __launch_bounds__(256, 2) void attend_flash_kernel(
       }
     }
   };
-  int xrun = -100;  // q8_0: X of this wave's staged dims
+  // q8_0: X with the slice's factors f (lane: key), and whether this lane's key
+  // stays out of the product: a half's factor is 11 bits, and down to 2^(X - 22)
+  // its products' low halves end at 2^-24
+  auto track = [&](float f, int& x) __attribute__((always_inline)) {
+    const float af = fabsf(f), fm = lanes::reduce<64>(af < INFINITY ? af : 0.0f, lanes::Max{});
+    if (fm > 0.0f) x = max(x, __builtin_amdgcn_frexp_expf(fm));
+    x = __builtin_amdgcn_readfirstlane(x);
+    return !(af < INFINITY) || (af > 0.0f && __builtin_amdgcn_frexp_expf(af) < x - 21);
+  };
+  int xrun = -100;  // X of this wave's staged dims
   auto store_v = [&](int buf) __attribute__((always_inline)) {
     if constexpr (Q8) {
-      const float fm = lanes::reduce<64>(fabsf(vfr), lanes::Max{});
-      if (fm > 0.0f) xrun = max(xrun, __builtin_amdgcn_frexp_expf(fm));
-      xrun = __builtin_amdgcn_readfirstlane(xrun);
+      // (what lies where no key is held may be another sequence's)
+      const float fv = (dead >> lane) & 1 ? 0.0f : half_bits_to_float(vfr);
+      const bool out = track(fv, xrun);
       if (lane == 0) vexp[wave] = xrun;
-      const _Float16 f = (_Float16)ldexpf(vfr, 8 - xrun);
+      if (out) left_out = 1;
+      const _Float16 f = (_Float16)(out ? 0.0f : ldexpf(fv, 8 - xrun));
       const fh2 f2 = {f, f};
 #pragma unroll
       for (int j = 0; j < PER; j++) {
@@ -269,6 +265,41 @@ __global__ __launch_bounds__(256, 2) void attend_flash_kernel(
       }
     }
   };
+
+  // the first slice on its way behind the queries, ahead of their conversion
+  load(kc, s0, kr, kfr);
+  load(vc, s0, vr, vfr);
+  __builtin_amdgcn_sched_barrier(0);
+
+  // The query, scaled by the power of two that brings its largest value to
+  // [2^14, 2^15) and split into three halves; scores are taken against |scale|
+  // log2(e), which takes the power back, the query carrying scale's sign.
+  float c2 = fabsf(scale) * kLog2e;
+  fh8 qf[3][D / 16];
+  {
+    float mx = 0.0f;
+#pragma unroll
+    for (int st = 0; st < D / 16; st++)
+#pragma unroll
+      for (int u = 0; u < 8; u++) mx = fmaxf(mx, fabsf(qraw[st][u >> 2][u & 3]));
+    mx = other_max(mx);
+    const int e = mx > 0.0f ? max(__builtin_amdgcn_frexp_expf(mx) - 15, -126) : 0;
+    c2 = ldexpf(c2, e);
+    const float sc = ldexpf(scale < 0.0f ? -1.0f : 1.0f, -e);
+#pragma unroll
+    for (int st = 0; st < D / 16; st++) {
+#pragma unroll
+      for (int u = 0; u < 8; u++) {
+        const float f = sc * qraw[st][u >> 2][u & 3];
+        const _Float16 h1 = (_Float16)f;
+        const float r1 = f - (float)h1;  // exact
+        const _Float16 h2 = (_Float16)r1;
+        qf[0][st][u] = h1;
+        qf[1][st][u] = h2;
+        qf[2][st][u] = (_Float16)(r1 - (float)h2);
+      }
+    }
+  }
 
   ff16 o[NT];
 #pragma unroll
@@ -401,13 +432,9 @@ __global__ __launch_bounds__(256, 2) void attend_flash_kernel(
       }
   };
 
-  if (s0 < s1) {
-    load(kc, s0, kr, kfr);
-    load(vc, s0, vr, vfr);
-    store_k(0);
-    store_v(0);
-    __syncthreads();
-  }
+  store_k(0);
+  store_v(0);
+  __syncthreads();
   for (int sl = s0; sl < s1; sl++) {
     const int buf = (sl - s0) & 1, base = sl * kSlice;
     const bool more = sl + 1 < s1;          // uniform
@@ -428,6 +455,53 @@ __global__ __launch_bounds__(256, 2) void attend_flash_kernel(
     if (Q8) __syncthreads();  // the one value buffer has been read
     if (more) store_v(1 - buf);
     __syncthreads();
+  }
+
+  // q8_0: the keys that were left out (the same ones: X runs as it did), added
+  // in float32 to the rows that they are live for.  Their weights are in l.
+  if constexpr (Q8) {
+    if (__builtin_expect(left_out, 0)) {
+      // (from the thread's index again, and the queries' power of two out of c2:
+      // kept through the loop they cost it six registers, which it spilled)
+      int tid = threadIdx.x;
+      asm volatile("" : "+v"(tid));
+      const int lane = tid & 63, h = lane >> 5, r = 32 * (tid >> 6) + (lane & 31);
+      const int t = t0 + r / group, head = kvh * group + r % group, cnt = t < tokens ? pos[t] + 1 : 0;
+      const int e = __builtin_amdgcn_frexp_expf(c2) - __builtin_amdgcn_frexp_expf(fabsf(scale) * kLog2e);
+      const float sc = ldexpf(scale < 0.0f ? -1.0f : 1.0f, -e);
+      const float* qr = q + (int64_t)min(t, tokens - 1) * q_stride + (int64_t)head * D + 8 * h;
+#pragma unroll
+      for (int dt = 0; dt < NT; dt++) {
+        int x = -100;
+        for (int sl = s0; sl < s1; sl++) {
+          const int cell = cell_of(sl, lane);
+          float f = __half2float(vc[row_of(cell) + (kvw >> 1) + ((kvh * D) >> 5) + dt]);
+          if (sl * kSlice + lane >= count || cell < 0) f = 0.0f;
+          for (uint64_t outs = __ballot(track(f, x)); outs; outs &= outs - 1) {
+            const int k = __builtin_ctzll(outs);
+            const int64_t row = row_of(__shfl(cell, k));
+            const int8_t* kb = (const int8_t*)(kc + row) + kvh * D + 8 * h;
+            const __half* kfac = kc + row + (kvw >> 1) + ((kvh * D) >> 5);
+            float s = 0.0f;
+#pragma nounroll
+            for (int st = 0; st < D / 16; st++) {
+              float b = 0.0f;
+              for (int u = 0; u < 8; u++) b = fmaf((float)kb[16 * st + u], sc * qr[16 * st + u], b);
+              s = fmaf(__half2float(kfac[st >> 1]), b, s);
+            }
+            s = other_sum(s);
+            const float p = __builtin_amdgcn_exp2f(fmaf(s - mc, c2, kLift));
+            const float fk = __shfl(f, k) * ldexpf(1.0f, 8 - xo[dt]);
+            const int8_t* vb = (const int8_t*)(vc + row) + kvh * D + 32 * dt + 4 * h;
+            if (sl * kSlice + k < cnt) {
+#pragma unroll
+              for (int j = 0; j < 16; j++)
+                o[dt][j] = fmaf(p, (float)vb[8 * (j >> 2) + (j & 3)] * fk, o[dt][j]);
+            }
+          }
+        }
+      }
+    }
   }
 
   l = other_sum(l);

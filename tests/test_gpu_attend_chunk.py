@@ -124,3 +124,72 @@ def test_chunk_query_of_any_size(form, dims, power):
         block.device_layer(ctx, l, xd, kd, vd, 0, posd, count, tokens, form=f)
         outs.append(xd.cpu())
     assert torch.isfinite(outs[0]).all() and torch.equal(outs[0], outs[1])
+
+
+@pytest.mark.parametrize("dims", [(512, 256, 8, 2, 64), (1024, 256, 8, 1, 128), (256, 256, 4, 4, 64)])
+@pytest.mark.parametrize("paged", [False, True])
+@pytest.mark.parametrize("infinite", [False, True])
+def test_q8_value_factors_of_any_range(dims, paged, infinite):
+    """Value factors 2^28 apart, or infinite, at positions that only the chunk's
+    last token reaches (and in cell 0 of the pool, where positions that are not
+    held look): the earlier tokens keep every bit, and the last one, which sums
+    both sizes, is right too.  The gate is the layer's own."""
+    from molla_amd import block, gpu
+    from tests.test_gpu_kernels import q8_decode, q8_rows
+    ctx = gpu.DeviceContext(0)
+    spec = spec_of(*dims)
+    host = make_layer_weights(spec, 29)
+    host["attn_norm"] = (host["attn_norm"] * 0.05).astype(np.float32)
+    kind, r, c, blob = host["down"]
+    host["down"] = (kind, r, c, np.zeros_like(blob))
+    bs, layer = device_layer_from(host, spec)
+    kvw, count = bs.kv_width(), 200
+    row = gpu.cache_row(gpu.CACHE_Q8, kvw)
+    pos = np.array(list(range(60, 71)) + [count - 1])  # 11 tokens, and one past rows that lie there
+    k, v = (synth.normal(count * kvw, 98 + i).numpy().reshape(count, kvw) for i in (0, 1))
+    v *= np.float32(2.0 ** -8)
+    big = np.arange(count) % 7 == 3
+    big[:71] = False
+    v[big] *= np.float32(2.0 ** 28)
+    rows = [q8_rows(a, kvw).reshape(count, row) for a in (k, v)]
+    if infinite:
+        rows[1][big, kvw // 2:] = 0x7c00
+    held = np.ones(count, bool)
+    held[5:60:6] = False
+    if not paged:
+        held[:] = True
+    order = 1 + np.random.default_rng(4).permutation(count + 3)[:count].astype(np.int32)
+    x = synth.normal(pos.size * bs.width, 101).numpy()
+    xd = torch.from_numpy(x.copy()).cuda()
+    posd = torch.from_numpy(pos.astype(np.int32)).cuda()
+
+    def dev(a):
+        return torch.from_numpy(np.ascontiguousarray(a).view(np.int16)).view(torch.float16).cuda()
+
+    if paged:
+        pools = [np.zeros((count + 4, row), np.uint16) for _ in rows]
+        for p, a in zip(pools, rows):
+            p[order] = a
+            p[0, :kvw // 2] = 0x0101
+            p[0, kvw // 2:] = 0x7c00
+        kd, vd = (dev(p.reshape(-1)) for p in pools)
+        idx = torch.from_numpy(np.where(held, order, -1).astype(np.int32)).cuda()
+        block.device_layer_paged(ctx, layer, xd, kd, vd, idx, 0, posd, count, pos.size, form=gpu.CACHE_Q8)
+    else:
+        order = np.arange(count)
+        kd, vd = (dev(a.reshape(-1)) for a in rows)
+        block.device_layer(ctx, layer, xd, kd, vd, 0, posd, count, pos.size, form=gpu.CACHE_Q8)
+    ctx.synchronize()
+    got = [c.cpu().view(torch.int16).numpy().view(np.uint16).reshape(-1, row)[order] for c in (kd, vd)]
+    with np.errstate(invalid="ignore"):  # 0 x infinity, in rows that are not looked at
+        got = [q8_decode(g.reshape(-1), kvw, count) for g in got]
+    keep = []
+    L = oracle.make_layer(spec, host, keep)
+    for i in (0, 1, 10) + (() if infinite else (11,)):
+        kept = [j for j in range(pos[i]) if held[j]]
+        slot = len(kept)
+        kr, vr = (np.concatenate([g[kept], np.zeros((1, kvw), np.float32)]).astype(np.float32).reshape(-1) for g in got)
+        xr = x.reshape(pos.size, -1)[i].copy()
+        bound = layer_gate(spec, host, xr, kr, vr, slot)
+        oracle.layer_step(L, xr, kr, vr, slot, int(pos[i]), f16_store=False, q8_store=True, threads=8)
+        assert_layer_close(xd.cpu().numpy().reshape(pos.size, -1)[i], xr, bound, f"token {i}:")

@@ -134,3 +134,56 @@ def test_large_and_small_queries(form, size, keys):
                       gpu.CACHE_Q8 if form == "q8" else gpu.CACHE_F16)
     want = oracle.attend(heads, kv, hd, scale, q, host[0], host[1], count)
     assert np.abs(out.cpu().numpy() - want).max() <= 1e-5 * np.abs(want).max()
+
+
+@pytest.mark.parametrize("heads,kv,hd", [(8, 2, 128), (8, 1, 64)])
+def test_q8_value_factors_of_any_range(heads, kv, hd):
+    """Values 2^28 apart in the same block of 32: keys of large ones with
+    weights of e^-40 leave the others their bits."""
+    from molla_amd import gpu
+    from tests.test_gpu_kernels import q8_decode, q8_rows
+    ctx = gpu.DeviceContext(0)
+    count, kvw, scale = 700, kv * hd, np.float32(1 / np.sqrt(hd))
+    q = synth.normal(heads * hd, 84).numpy()
+    k = synth.normal(count * kvw, 85).numpy().reshape(count, kvw)
+    v = synth.normal(count * kvw, 86).numpy().reshape(count, kvw) * np.float32(2.0 ** -8)
+    big = np.arange(count) % 9 == 4
+    away = q.reshape(kv, -1, hd).sum(1).reshape(-1)  # every head of a group scores about -40 along it
+    k[big] = -away * np.float32(40 / (hd * scale))
+    v[big] *= np.float32(2.0 ** 28)
+    rows = [q8_rows(c, kvw) for c in (k, v)]
+    kd, vd = (torch.from_numpy(r.view(np.int16).copy()).view(torch.float16).cuda() for r in rows)
+    kh, vh = (q8_decode(r, kvw, count).reshape(-1) for r in rows)
+    out = torch.zeros(heads * hd, device="cuda")
+    gpu.device_attend(ctx, torch.from_numpy(q).cuda(), kd, vd, heads, kv, hd, float(scale), count, out, gpu.CACHE_Q8)
+    want = oracle.attend(heads, kv, hd, float(scale), q, kh, vh, count)
+    assert np.abs(out.cpu().numpy() - want).max() <= 1e-5 * np.abs(want).max()
+
+
+@pytest.mark.parametrize("tokens", [1, 3])
+@pytest.mark.parametrize("factor", [0x7c00, 0x7bff])
+def test_q8_cells_not_held_leave_no_trace(tokens, factor):
+    """Positions that are not held read cell 0, which is another sequence's: an
+    infinite or the largest factor there changes no bit."""
+    from molla_amd import block, gpu
+    from tests.test_gpu_layer import device_layer_from, make_layer_weights, spec_of
+    ctx = gpu.DeviceContext(0)
+    spec = spec_of(512, 512, 8, 2, 64)
+    bs, layer = device_layer_from(make_layer_weights(spec, 33), spec)
+    kvw, pos = bs.kv_width(), 300
+    row = gpu.cache_row(gpu.CACHE_Q8, kvw)
+    (k, v), _ = caches("q8", 1 + tokens * (pos + 1), kvw, 54)
+    index = 1 + torch.randperm(tokens * (pos + 1), generator=torch.Generator().manual_seed(5)).reshape(tokens, pos + 1)
+    index[:, 3:pos:5] = -1
+    index = index.to(torch.int32).cuda()
+    x = synth.normal(tokens * bs.width, 56).cuda()
+    posd = torch.full((tokens,), pos, dtype=torch.int32, device="cuda")
+    outs = []
+    for poison in (False, True):
+        xd, kd, vd = x.clone(), k.clone(), v.clone()
+        if poison:
+            for c in (kd, vd):
+                c[kvw // 2:row] = torch.tensor([factor] * (row - kvw // 2), dtype=torch.int16).view(torch.float16).cuda()
+        block.device_layer_paged(ctx, layer, xd, kd, vd, index, pos + 1, posd, pos + 1, tokens, form=gpu.CACHE_Q8)
+        outs.append(xd.cpu())
+    assert torch.isfinite(outs[0]).all() and torch.equal(outs[0], outs[1])
