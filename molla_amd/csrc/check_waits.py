@@ -12,6 +12,10 @@ moves a load ahead of the LDS load, or merges two into one, ends up with too few
 and the check fails.  Only global and buffer loads count as younger ones.  A
 label or a branch in between fails too: the order of the lines is then not the
 order of execution.
+
+m0 holds an LDS load's address, and the compiler does not know that the assembly
+writes it: it may appear only where a load sets it, with nothing but an s_nop
+before the load.
 """
 
 import re
@@ -19,11 +23,13 @@ import sys
 
 LDS_LOAD = re.compile(r"(global|buffer)_load_lds_|(global|buffer)_load_\S+\s.*\blds\b")
 LOAD = re.compile(r"(global|buffer)_load_")
+M0 = re.compile(r"\bm0\b")
 VMCNT = re.compile(r"vmcnt\((\d+)\)")
 
 
 def check(lines):
-    """(LDS loads seen, messages about those without a wait)."""
+    """(LDS loads seen, messages about what is wrong)."""
+    m0 = None  # the line that set m0 for the next LDS load
     pending = []  # [line number, younger loads] of LDS loads not known to have landed
     seen, bad = 0, []
 
@@ -37,6 +43,17 @@ def check(lines):
             if re.match(r"\.L\w+:", text):  # (a label that is jumped to)
                 fail(at, "a label")
             continue
+        if M0.search(text):
+            if not text.startswith("s_mov_b32 m0,") or m0 is not None:
+                bad.append(f"line {at}: m0 used by other code")
+            m0 = at
+            continue
+        if m0 is not None and not text.startswith("s_nop"):
+            if not LDS_LOAD.match(text):
+                bad.append(f"line {m0}: m0 set, and no LDS load after it")
+            m0 = None
+        elif LDS_LOAD.match(text):
+            bad.append(f"line {at}: an LDS load whose m0 was not set")
         if LDS_LOAD.match(text):
             for p in pending:
                 p[1] += 1

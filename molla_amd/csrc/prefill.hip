@@ -562,12 +562,13 @@ __global__ __launch_bounds__(WR * KS * 64, (WR * KS + 3) / 4) void prefill_kerne
       asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %1, %2"
                    :
                    : "s"(lds0 + buf * kStageBytes + kb * 1024), "v"(lane16), "s"(src)
-                   : "memory", "m0");
+                   : "memory");  // (m0 is a reserved register: naming it is only warned of)
     }
   };
   // Loads complete in order: with at most N younger ones in flight, the
   // transfer has landed.  N counts the loads issued after it, or fewer
-  // (check_waits.py looks the compiled code over for it in every build).
+  // (check_waits.py looks the compiled code over for it in every build, and that
+  // nothing else uses m0).
   auto wait_x = [&](auto nn) __attribute__((always_inline)) {
     constexpr int N = decltype(nn)::value;
     static_assert(N < 16, "one field of s_waitcnt's encoding");

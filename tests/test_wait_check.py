@@ -46,6 +46,8 @@ def test_covered_loads_pass():
     ("a load moved ahead of the transfer", GOOD.replace(LOAD, "").replace("	s_mov_b32 m0, s35\n", LOAD + "	s_mov_b32 m0, s35\n")),
     ("a load moved behind the wait", GOOD.replace(LOAD, "").replace("	s_barrier\n", LOAD + "	s_barrier\n")),
     ("a store is no load", GOOD.replace(LOAD, "	global_store_dword v[4:5], v6, off\n")),
+    ("m0 read by other code", GOOD.replace("	ds_read", "	s_add_u32 s3, m0, s4\n	ds_read")),
+    ("a load on the m0 of another", GOOD.replace("	s_mov_b32 m0, s36\n", "")),
     ("the wait is gone", GOOD.replace("	s_waitcnt vmcnt(2)\n", "")),
     ("a branch round the wait", GOOD.replace("	s_waitcnt vmcnt(2)\n", "	s_cbranch_execz .LBB0_2\n	s_waitcnt vmcnt(2)\n.LBB0_2:\n")),
 ])
