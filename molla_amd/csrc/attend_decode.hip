@@ -4,18 +4,23 @@
 // attend_kernel's `form`), GQA with up to 8 query heads a key head, head_dim
 // 64 or 128; the split and the fold of gpu_ops.mojo:929 / 1104.
 //
-// A block takes a share of one (key head, token)'s keys; each of its four
-// waves walks every fourth 32-key run of the share by itself, with a running
-// maximum and sum in registers and its own LDS rows for the values (no block
-// barrier until the waves' results are folded at the end), and sends for the
-// next run's keys and values as soon as it has used this one's.  The number of
-// shares fills the chip and stays at 64, so a long context costs a few partial
-// results a head and not one a 64-key slice.  us for the shares + the fold (the
-// 64-key slices' kernel + merge before), 32 heads of 128 over 8 key heads:
-// 32768 keys f16, cold, 34.6 + 4.6 (34.4 + 21.4: 134 MB at 3.9 TB/s, near the
-// read rate); 4097 keys 7.7 + 3.6 (6.7 + 6.0: latency, one run a wave); 8
-// sequences of 4700 keys, paged q8_0, 34.7 + 4.7 (51.1 + 7.3: the loads' latency
-// at two waves a SIMD, 2.4 TB/s).
+// A block takes a share of one (key head, token)'s keys: every shares-th step of
+// 32 keys a wave.  Each of its two or four waves walks its 32-key runs by itself,
+// with a running maximum and sum in registers and its own LDS rows for the values
+// (no block barrier until the waves' results are folded at the end), and sends for
+// the next run's keys and values as soon as it has used this one's.  The number of
+// shares (decode_attend_plan) is the one with the fewest runs in line on a compute
+// unit and stays at 64, so a long context costs a few partial results a head and
+// not one a 64-key slice.
+//
+// What bounds it: to about 1000 keys a chain of latencies (of ~7500 cycles of a
+// block with one run a wave the position takes ~1000, the keys ~2500, the softmax
+// ~800, the weighted values ~700, the fold ~1000); beyond, the loads: a layer's
+// attention over 32768 keys f16, cold, moves 134 MB in 34 us.  us of a layer of
+// width 256 with 32 heads of 128 over 8 key heads, caches cold (a 64-key slice a
+// block and a merge of the slices -> now): one sequence of 300 keys 26.2 -> 26.4, of
+// 2304 28.6 -> 28.3, of 32768 71.2 -> 51.1; eight of 300 50.9 -> 50.5, of 2304 64.7 ->
+// 64.6, of 8000 102.7 -> 96.4; eight of 6000 and less, paged q8_0, 101.5 -> 79.5.
 //
 //   S^T = K Q^T, keys as rows (read straight from the cache) and queries as
 //   columns: a lane's 8 scores belong to its own query, the softmax takes two
@@ -52,9 +57,7 @@ typedef uint32_t du4 __attribute__((ext_vector_type(4)));
 typedef uint32_t du2 __attribute__((ext_vector_type(2)));
 
 constexpr int kRun = 32;            // keys a wave takes at a time
-constexpr int kWaves = 4;           // waves a block
-constexpr int kStep = kRun * kWaves;  // keys a block takes at a time
-constexpr int kMaxShares = 64;
+constexpr int kMaxShares = 64;      // of a (key head, token)'s keys
 constexpr float kLift = 14.0f;      // P in [0, 2^14]: see attend_flash.hip
 constexpr float kLog2e = 1.44269504088896340736f;
 
@@ -93,31 +96,41 @@ __device__ __forceinline__ dh8 int8_halves(uint32_t x, uint32_t y) {
   return __builtin_bit_cast(dh8, r);
 }
 
-// The grid is (shares, kv_heads, tokens); share s takes the s-th part of the
-// 128-key steps that the token's own count has (a device value: the host
-// knows only the context) and writes each head's unnormalised sum with
-// (maximum, sum) in base 2 to slot (token, head, share); (0, 0) for no keys.
-template <int D, bool Q8, bool PAGED>
-__global__ __launch_bounds__(64 * kWaves, 2) void attend_decode_kernel(
+// The grid is (shares, kv_heads, tokens); share s takes every shares-th step of
+// 32 keys a wave of the token's own count (a device value: the host knows only
+// the context), starting at the s-th, and writes each head's unnormalised sum
+// with (maximum, sum) in base 2 to slot (token, head, share); (0, 0) for no
+// keys.
+template <int D, bool Q8, bool PAGED, int W>
+__global__ __launch_bounds__(64 * W, 2) void attend_decode_kernel(
     const float* __restrict__ q, int64_t q_stride, const __half* __restrict__ kc, const __half* __restrict__ vc,
     int64_t cache_stride, int row_halves, int heads, int kv_heads, int group, float scale,
     const int32_t* __restrict__ pos, int count_host, const int32_t* __restrict__ kv_index, int64_t index_stride,
     float* __restrict__ part_acc, float* __restrict__ part_ml) {
+  constexpr int kStep = kRun * W;  // keys a block takes at a time
   constexpr int KS = D / 32, NT = D / 16, PIECES = D / 8;
   constexpr int kFac = Q8 ? 2 * KS * kRun : 1;             // floats: factors of a run's keys and values
   constexpr int kWaveBytes = kRun * D * 2;                 // a run's values as halves
-  __shared__ __align__(16) uint8_t vs[kWaves][kWaveBytes];  // afterwards the waves' sums
-  __shared__ __align__(16) float fac[kWaves][kFac];
-  __shared__ float wml[kWaves][2][16];
+  __shared__ __align__(16) uint8_t vs[W][kWaveBytes];  // afterwards the waves' sums
+  __shared__ __align__(16) float fac[W][kFac];
+  __shared__ __align__(16) float wml[2][8][W];  // (maximum, sum) of a head, the waves side by side
   static_assert(8 * D * 4 <= kWaveBytes, "a wave's sums of 8 heads in place of its values");
   const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
   const int lm = lane & 15, lk = lane >> 4;
   const int share = blockIdx.x, shares = gridDim.x, kvh = blockIdx.y, t = blockIdx.z;
-  const int count = pos ? pos[t] + 1 : count_host;
-  const int steps = (count + kStep - 1) / kStep, per = (steps + shares - 1) / shares;
-  const int s0 = share * per, s1 = min(s0 + per, steps);
   const int64_t slot0 = ((int64_t)t * heads + (int64_t)kvh * group) * shares + share;
-  if (s0 >= s1) {
+  const int count = pos ? pos[t] + 1 : count_host;
+  // the queries, first in line, also ahead of the position: column lm (past the
+  // group, the last one)
+  const float* qr = q + (int64_t)t * q_stride + ((int64_t)kvh * group + min(lm, group - 1)) * D + 8 * lk;
+  df4 qraw[KS][2];
+#pragma unroll
+  for (int ks = 0; ks < KS; ks++) {
+    qraw[ks][0] = *(const df4*)(qr + 32 * ks);
+    qraw[ks][1] = *(const df4*)(qr + 32 * ks + 4);
+  }
+  __builtin_amdgcn_sched_barrier(0);
+  if (share * kStep >= count) {
     if (tid < group) *(float2*)(part_ml + (slot0 + (int64_t)tid * shares) * 2) = make_float2(0.0f, 0.0f);
     return;
   }
@@ -135,15 +148,6 @@ __global__ __launch_bounds__(64 * kWaves, 2) void attend_decode_kernel(
     const int cell = PAGED ? max(__shfl(cells, r), 0) : min(key + r, count - 1);
     return seq + (int64_t)cell * row_halves;
   };
-
-  // the queries, first in line: column lm (past the group, the last one)
-  const float* qr = q + (int64_t)t * q_stride + ((int64_t)kvh * group + min(lm, group - 1)) * D + 8 * lk;
-  df4 qraw[KS][2];
-#pragma unroll
-  for (int ks = 0; ks < KS; ks++) {
-    qraw[ks][0] = *(const df4*)(qr + 32 * ks);
-    qraw[ks][1] = *(const df4*)(qr + 32 * ks + 4);
-  }
 
   // a run's keys (lane: key lm of each 16-key tile, its values 32 ks + 8 lk ..
   // +8), values (16-byte pieces of its rows) and q8_0 factors (lane: key
@@ -185,12 +189,13 @@ __global__ __launch_bounds__(64 * kWaves, 2) void attend_decode_kernel(
   // this wave's maximum in base 2 and sum
   float m2 = -INFINITY, l = 0.0f;
 
-  int key0 = s0 * kStep + kRun * wave;
+  const int stride = shares * kStep;  // to this wave's next run
+  int key0 = share * kStep + kRun * wave;
   if (key0 < count) {  // (uniform over the wave; else it has no keys)
     int cells = cells_of(key0);
     load_k(key0, cells);
     load_v(key0, cells);
-    int cells_next = cells_of(key0 + kStep);
+    int cells_next = cells_of(key0 + stride);
     __builtin_amdgcn_sched_barrier(0);
 
     // the queries as B fragments: column lm (zero past the group), each scaled by
@@ -213,11 +218,11 @@ __global__ __launch_bounds__(64 * kWaves, 2) void attend_decode_kernel(
         for (int u = 0; u < 8; u++) {
           const float f = qraw[ks][u >> 2][u & 3] * sc;
           const _Float16 h1 = (_Float16)f;
-          const float r1 = f - (float)h1;  // exact
+          const float r1 = fmaf((float)h1, -1.0f, f);  // exact (as an fma it takes the half as it is)
           const _Float16 h2 = (_Float16)r1;
           qf[0][ks][u] = h1;
           qf[1][ks][u] = h2;
-          qf[2][ks][u] = (_Float16)(r1 - (float)h2);
+          qf[2][ks][u] = (_Float16)fmaf((float)h2, -1.0f, r1);
         }
       }
     }
@@ -235,8 +240,7 @@ __global__ __launch_bounds__(64 * kWaves, 2) void attend_decode_kernel(
     }
     float mc = -1e30f;  // the running maximum, of the scores before c2
 
-    for (int sl = s0; sl < s1; sl++, key0 += kStep) {
-      if (key0 >= count) break;  // (uniform over the wave: no keys left for it)
+    for (; key0 < count; key0 += stride) {  // (uniform over the wave)
       uint32_t held = 0xffffffffu;
       if constexpr (PAGED) held = (uint32_t)__ballot(cells >= 0);
       const int nk = min(kRun, count - key0);
@@ -274,8 +278,8 @@ __global__ __launch_bounds__(64 * kWaves, 2) void attend_decode_kernel(
             for (int h = 0; h < 3; h++) s[a] = mfma16(__builtin_bit_cast(dh8, kw[a][ks]), qf[h][ks], s[a]);
         }
       }
-      const bool more = key0 + kStep < count && sl + 1 < s1;  // uniform
-      if (more) load_k(key0 + kStep, cells_next);
+      const bool more = key0 + stride < count;  // uniform
+      if (more) load_k(key0 + stride, cells_next);
 
       // running maximum and weights of this lane's keys 16 a + 4 lk + i
       const uint32_t mine = held >> (4 * lk);
@@ -290,13 +294,13 @@ __global__ __launch_bounds__(64 * kWaves, 2) void attend_decode_kernel(
       m = across(m, lanes::Max{});
       const float mn = fmaxf(mc, m);
       const bool rose = mn != mc;
-      if (__any(rose)) {
+      if (__any(rose && l != 0.0f)) {  // (else there is nothing yet)
         const float f = __builtin_amdgcn_exp2f((mc - mn) * c2);
         l *= f;
 #pragma unroll
         for (int dt = 0; dt < NT; dt++) o[dt] *= f;
-        mc = mn;
       }
+      mc = mn;
       float p[8];
 #pragma unroll
       for (int a = 0; a < 2; a++)
@@ -328,9 +332,9 @@ __global__ __launch_bounds__(64 * kWaves, 2) void attend_decode_kernel(
           for (int a = 0; a < 2; a++) fv[b][a] = *(const df4*)(fl + KS * kRun + b * kRun + 16 * a + 4 * lk);
       }
       asm volatile("" ::: "memory");  // (a wave's LDS operations complete in order)
-      if (more) load_v(key0 + kStep, cells_next);
+      if (more) load_v(key0 + stride, cells_next);
       cells = cells_next;
-      cells_next = cells_of(key0 + 2 * kStep);
+      cells_next = cells_of(key0 + 2 * stride);
 
       dh8 ph, pl;
       if constexpr (!Q8) {
@@ -392,7 +396,10 @@ __global__ __launch_bounds__(64 * kWaves, 2) void attend_decode_kernel(
     if (l != 0.0f) m2 = mc * c2;  // (no key held: no part in the fold)
   }
 
-  // fold the waves: their sums (in place of the values) and (maximum, sum)
+  // fold the waves: their sums (in place of the values) and (maximum, sum), four
+  // dims a thread and every read sent for at once (a dim at a time, with the
+  // weights found again for each, this took 3700 of a short context's 10000
+  // cycles)
   float* wo = (float*)&vs[0][0];  // [wave][group][D]
   __syncthreads();
   if (lm < group) {
@@ -402,25 +409,33 @@ __global__ __launch_bounds__(64 * kWaves, 2) void attend_decode_kernel(
       *(df4*)(wo + (wave * group + lm) * D + 16 * dt + 4 * lk) = o[dt];
     }
     if (lk == 0) {
-      wml[wave][0][lm] = m2;
-      wml[wave][1][lm] = l;
+      wml[0][lm][wave] = m2;
+      wml[1][lm][wave] = l;
     }
   }
   __syncthreads();
-  for (int i = tid; i < group * D; i += 64 * kWaves) {
-    const int g = i / D, d = i - g * D;
-    float m = -3e38f;
+  for (int i = tid; i < group * (D / 4); i += 64 * W) {
+    const int g = i / (D / 4), d = 4 * (i % (D / 4));
+    df4 a[W];
+    float mw[W], lw[W], m = -3e38f;
 #pragma unroll
-    for (int w = 0; w < kWaves; w++) m = fmaxf(m, wml[w][0][g]);
-    float v = 0.0f, sum = 0.0f;
+    for (int w = 0; w < W; w++) {
+      a[w] = *(const df4*)(wo + (w * group + g) * D + d);
+      mw[w] = wml[0][g][w];
+      lw[w] = wml[1][g][w];
+      m = fmaxf(m, mw[w]);
+    }
+    df4 v = {0.0f, 0.0f, 0.0f, 0.0f};
+    float sum = 0.0f;
 #pragma unroll
-    for (int w = 0; w < kWaves; w++) {
-      const float f = __builtin_amdgcn_exp2f(wml[w][0][g] - m);
-      v = fmaf(wo[(w * group + g) * D + d], f, v);
-      sum = fmaf(wml[w][1][g], f, sum);
+    for (int w = 0; w < W; w++) {
+      const float f = __builtin_amdgcn_exp2f(mw[w] - m);
+#pragma unroll
+      for (int e = 0; e < 4; e++) v[e] = fmaf(a[w][e], f, v[e]);
+      sum = fmaf(lw[w], f, sum);
     }
     const int64_t slot = slot0 + (int64_t)g * shares;
-    part_acc[slot * D + d] = v;
+    *(df4*)(part_acc + slot * D + d) = v;
     if (d == 0) *(float2*)(part_ml + slot * 2) = make_float2(m, sum);
   }
 }
@@ -431,32 +446,57 @@ bool decode_attend_fits(int32_t group, int32_t head_dim) {
   return (group == 1 || group == 2 || group == 4 || group == 8) && (head_dim == 64 || head_dim == 128);
 }
 
-// Shares of the keys: about four blocks a compute unit, at most one a 128-key
-// step of the context and 64 (the fold takes them in one round).
-int decode_attend_shares(int32_t kv_heads, int32_t tokens, int32_t max_count) {
-  const int steps = (max_count + kStep - 1) / kStep;
-  const int want = (4 * cu_count() + kv_heads * tokens - 1) / (kv_heads * tokens);
-  return std::max(1, std::min({want, steps, kMaxShares}));
+// Two-wave blocks while every 64 keys of the context can have a compute unit of
+// their own: one unit takes in about 64 bytes a cycle, so that a short context is
+// better spread (us of a layer of width 256, two / four waves: 300 keys 26.3 / 27.4,
+// 700 in a context of 1024 26.9 / 27.7, 1100 in 2048 27.6 / 28.0, four sequences of
+// 300 in 512 38.3 / 39.6, two of 600 in 1024, q8_0, 40.3 / 39.8; past the line eight
+// of 300 in 512 51.4 / 50.5, one of 2304 28.7 / 28.2).
+//
+// Shares: a compute unit with n blocks of r runs a wave takes n r runs' time, whether
+// the blocks run side by side or in turn, and about a quarter of a run's for each
+// block (us as above; 2304 keys, 18 steps, 32 pairs of a token and a key head: 6
+// shares of 3 are 192 blocks and 46.1, 9 of 2 are 288 and 49.3, 18 of 1 are 576 and
+// 46.9; 64 pairs: 4 shares 64.6, 6 64.8, 8 66.3, 16 69.9).  Of the equal ones the
+// fewest.  q8_0's loads wait on more arithmetic, so that one block a unit is a
+// sixteenth slower than that (eight paged sequences of 6000: 4 shares 87.4, 8 82.0,
+// 16 87.0).  At most 64, which the fold takes in one round.
+DecodePlan decode_attend_plan(int32_t kv_heads, int32_t tokens, int32_t max_count, bool q8) {
+  const int64_t pairs = (int64_t)kv_heads * tokens, cus = cu_count();
+  const int waves = pairs * ((max_count - 1) / (2 * kRun) + 1) <= cus ? 2 : 4;
+  const int64_t steps = (max_count - 1) / (kRun * waves) + 1;
+  DecodePlan best{waves, 1};
+  int64_t least = INT64_MAX;
+  for (int n = 1; n <= std::min<int64_t>(steps, kMaxShares); n++) {
+    const int64_t deep = (n * pairs + cus - 1) / cus;
+    int64_t cost = 16 * deep * (4 * ((steps + n - 1) / n) + 1);
+    if (q8 && deep == 1) cost += cost / 16;
+    if (cost < least) best.shares = n, least = cost;
+  }
+  return best;
 }
 
 int launch_attend_decode(hipStream_t s, const float* q, int64_t q_stride, const uint16_t* k_cache,
                          const uint16_t* v_cache, int64_t cache_stride, int32_t heads, int32_t kv_heads,
-                         int32_t head_dim, float scale, const int32_t* pos, int32_t count_host, int32_t shares,
+                         int32_t head_dim, float scale, const int32_t* pos, int32_t count_host, DecodePlan plan,
                          int32_t tokens, float* part_acc, float* part_ml, int32_t form, const int32_t* kv_index,
                          int64_t index_stride) {
   const int row = cache_row(form, kv_heads * head_dim);
-  const dim3 grid(shares, kv_heads, tokens);
-#define MI_DEC(DD, Q, P)                                                                                         \
-  hipLaunchKernelGGL((attend_decode_kernel<DD, Q, P>), grid, dim3(64 * kWaves), 0, s, q, q_stride,                 \
+  const dim3 grid(plan.shares, kv_heads, tokens);
+#define MI_DEC_W(DD, Q, P, W)                                                                                      \
+  hipLaunchKernelGGL((attend_decode_kernel<DD, Q, P, W>), grid, dim3(64 * W), 0, s, q, q_stride,                   \
                      (const __half*)k_cache, (const __half*)v_cache, cache_stride, row, heads, kv_heads,           \
                      heads / kv_heads, scale, pos, count_host, kv_index, index_stride, part_acc, part_ml)
+#define MI_DEC(DD, Q, P)                              \
+  if (plan.waves == 4) MI_DEC_W(DD, Q, P, 4);         \
+  else MI_DEC_W(DD, Q, P, 2);
 #define MI_DEC_F(DD)                         \
   if (form == MI_CACHE_Q8) {                 \
-    if (kv_index) MI_DEC(DD, true, true);    \
-    else MI_DEC(DD, true, false);            \
+    if (kv_index) { MI_DEC(DD, true, true) }    \
+    else { MI_DEC(DD, true, false) }            \
   } else {                                   \
-    if (kv_index) MI_DEC(DD, false, true);   \
-    else MI_DEC(DD, false, false);           \
+    if (kv_index) { MI_DEC(DD, false, true) }   \
+    else { MI_DEC(DD, false, false) }           \
   }
   if (head_dim == 64) {
     MI_DEC_F(64)
@@ -465,6 +505,7 @@ int launch_attend_decode(hipStream_t s, const float* q, int64_t q_stride, const 
   }
 #undef MI_DEC_F
 #undef MI_DEC
+#undef MI_DEC_W
   return hip_check(hipGetLastError(), "attend_decode launch");
 }
 

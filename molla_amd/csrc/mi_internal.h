@@ -258,12 +258,16 @@ int launch_attend(hipStream_t s, const float* q, int64_t q_stride, const uint16_
 // Decode attention at head widths 64 and 128, either cache form
 // (attend_decode.hip): each token's keys in `shares` parts, whose (maximum,
 // sum) in base 2 and values go to part_ml / part_acc slot (token, head, share);
-// a share without keys leaves the sum 0 and no values.
+// a share without keys leaves the sum 0 and no values.  Never more shares than
+// the context has 64-key slices (launch_attend's workspace).
 bool decode_attend_fits(int32_t group, int32_t head_dim);
-int32_t decode_attend_shares(int32_t kv_heads, int32_t tokens, int32_t max_count);
+struct DecodePlan {
+  int32_t waves, shares;  // of a block; of the keys
+};
+DecodePlan decode_attend_plan(int32_t kv_heads, int32_t tokens, int32_t max_count, bool q8);
 int launch_attend_decode(hipStream_t s, const float* q, int64_t q_stride, const uint16_t* k_cache,
                          const uint16_t* v_cache, int64_t cache_stride, int32_t heads, int32_t kv_heads,
-                         int32_t head_dim, float scale, const int32_t* pos, int32_t count_host, int32_t shares,
+                         int32_t head_dim, float scale, const int32_t* pos, int32_t count_host, DecodePlan plan,
                          int32_t tokens, float* part_acc, float* part_ml, int32_t form, const int32_t* kv_index,
                          int64_t index_stride);
 // One sequence's chunk of more than kMaxTokens tokens at head widths 64 and

@@ -44,6 +44,84 @@ def test_decode_attention_edges(form, heads, kv, hd, count):
 
 
 @pytest.mark.parametrize("form", ["f16", "q8"])
+@pytest.mark.parametrize("heads,kv,hd", [(2, 2, 128), (16, 2, 64)])
+def test_several_steps_a_share(form, heads, kv, hd):
+    """20000 keys are 157 steps of a block's 128: three a share, the last of
+    them short."""
+    test_decode_attention_edges(form, heads, kv, hd, 20000)
+
+
+@pytest.mark.parametrize("form", ["f16", "q8"])
+@pytest.mark.parametrize("heads,kv,hd", [(16, 8, 64), (8, 8, 128)])
+@pytest.mark.parametrize("tokens", [3, 8])
+def test_paged_steps(form, heads, kv, hd, tokens):
+    """Sequences of unequal length, many steps a share: rows in the cells of a
+    pool, in no order, give the contiguous caches' result to the bit; with some
+    positions not held, the oracle's over the rows that are (the gate of
+    tests/test_gpu_layer.py)."""
+    from molla_amd import block, gpu
+    from tests.test_gpu_kernels import q8_decode
+    from tests.test_gpu_layer import assert_layer_close, device_layer_from, layer_gate, make_layer_weights, spec_of
+    ctx = gpu.DeviceContext(0)
+    f = gpu.CACHE_Q8 if form == "q8" else gpu.CACHE_F16
+    spec = spec_of(256, 256, heads, kv, hd)
+    host = make_layer_weights(spec, 35)
+    host["attn_norm"] = (host["attn_norm"] * 0.05).astype(np.float32)  # scores of a model's size
+    kind, r, c, blob = host["down"]
+    host["down"] = (kind, r, c, np.zeros_like(blob))  # (no MLP, which magnifies a last bit)
+    bs, layer = device_layer_from(host, spec)
+    kvw, length = bs.kv_width(), 2600
+    row = gpu.cache_row(f, kvw)
+    (k, v), _ = caches(form, tokens * length, kvw, 64)
+    pos = [length - 1 - 290 * t for t in range(tokens)]
+    posd = torch.tensor(pos, dtype=torch.int32, device="cuda")
+    x = synth.normal(tokens * bs.width, 66).cuda()
+
+    def contiguous(ks, vs, at):
+        xd, kd, vd = x.clone(), ks.clone(), vs.clone()
+        block.device_layer(ctx, layer, xd, kd, vd, length * row, at, length, tokens, form=f)
+        return xd.cpu()
+
+    def paged(held):
+        order = torch.randperm(tokens * length, generator=torch.Generator().manual_seed(6))
+        pools = []
+        for c in (k, v):
+            pool = torch.zeros(tokens * length, row, dtype=torch.float16, device="cuda")
+            pool[order.cuda()] = c.reshape(-1, row)
+            pools.append(pool.reshape(-1))
+        index = torch.where(held, order.reshape(tokens, length), -1).to(torch.int32).cuda()
+        xd = x.clone()
+        block.device_layer_paged(ctx, layer, xd, *pools, index, length, posd, length, tokens, form=f)
+        return xd.cpu()
+
+    held = torch.ones(tokens, length, dtype=torch.bool)
+    assert torch.equal(paged(held), contiguous(k, v, posd))
+
+    held[:, 5::9] = False
+    for t in range(tokens):
+        held[t, pos[t]] = True
+    got = paged(held)
+    keep = []
+    L = oracle.make_layer(spec, host, keep)
+
+    def floats(c):
+        a = c.cpu().view(torch.int16).numpy().view(np.uint16)
+        n = a.size // row
+        if form == "q8":
+            return q8_decode(a, kvw, n).reshape(n, kvw)
+        return a.view(np.float16).astype(np.float32).reshape(n, kvw)
+
+    for t in (0, tokens - 1):
+        rows = [j for j in range(pos[t]) if held[t, j]]
+        kr, vr = (np.concatenate([floats(c.reshape(tokens, length, row)[t])[rows], np.zeros((1, kvw), np.float32)])
+                  .astype(np.float32).reshape(-1) for c in (k, v))
+        xr = x.cpu().numpy().reshape(tokens, -1)[t].copy()
+        bound = layer_gate(spec, host, xr, kr, vr, len(rows))
+        oracle.layer_step(L, xr, kr, vr, len(rows), pos[t], f16_store=form != "q8", q8_store=form == "q8", threads=8)
+        assert_layer_close(got.numpy().reshape(tokens, -1)[t], xr, bound, f"sequence {t}:")
+
+
+@pytest.mark.parametrize("form", ["f16", "q8"])
 def test_scores_of_1e8(form):
     """Scores whose rounding is worth several powers of two of a weight: the
     largest weight stays 1.  Neighbouring scores lie 1e5 apart and more, so the
@@ -88,6 +166,36 @@ def test_context_longer_than_the_position(form, tokens):
         outs.append(xd.cpu().double())
     assert torch.isfinite(outs[1]).all()
     assert (outs[0] - outs[1]).norm() <= 1e-5 * outs[0].norm()
+
+
+@pytest.mark.parametrize("form", ["f16", "q8"])
+@pytest.mark.parametrize("dims", [(256, 256, 8, 2, 64), (256, 256, 16, 2, 128), (256, 256, 4, 4, 128)])
+def test_block_sizes(form, dims):
+    """Eight sequences that end at the edges of a run and of a step, in a context
+    that gives every 64 keys a compute unit (blocks of two waves) and in one
+    that does not (four): the same within the rounding of sums in another
+    order."""
+    from molla_amd import block, gpu
+    from tests.test_gpu_layer import device_layer_from, make_layer_weights, spec_of
+    ctx = gpu.DeviceContext(0)
+    f = gpu.CACHE_Q8 if form == "q8" else gpu.CACHE_F16
+    bs, layer = device_layer_from(make_layer_weights(spec_of(*dims), 37), spec_of(*dims))
+    pos = [0, 30, 31, 32, 63, 127, 128, 299]
+    kvw, length, tokens = bs.kv_width(), 300, len(pos)
+    row = gpu.cache_row(f, kvw)
+    (k, v), _ = caches(form, tokens * length, kvw, 68)
+    x = synth.normal(tokens * bs.width, 69).cuda()
+    posd = torch.tensor(pos, dtype=torch.int32, device="cuda")
+    outs = []
+    for context in (length, 20000):
+        # (the same rows, the longer cache's padded with ones that no position reaches)
+        kd, vd = (torch.cat([c.reshape(tokens, length * row), torch.zeros(tokens, (context - length) * row,
+                                                                         dtype=c.dtype, device="cuda")], 1).reshape(-1)
+                  for c in (k, v))
+        xd = x.clone()
+        block.device_layer(ctx, layer, xd, kd, vd, context * row, posd, context, tokens, form=f)
+        outs.append(xd.cpu().double().reshape(tokens, -1))
+    assert ((outs[0] - outs[1]).norm(dim=1) <= 1e-5 * outs[0].norm(dim=1)).all()
 
 
 @pytest.mark.parametrize("form", ["f16", "q8"])
