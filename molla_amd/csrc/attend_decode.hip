@@ -58,7 +58,7 @@ typedef uint32_t du2 __attribute__((ext_vector_type(2)));
 
 constexpr int kRun = 32;            // keys a wave takes at a time
 constexpr int kMaxShares = 64;      // of a (key head, token)'s keys
-constexpr float kLift = 14.0f;      // P in [0, 2^14]: see attend_flash.hip
+constexpr float kLift = 16384.0f;   // of P when it is split: see attend_flash.hip
 constexpr float kLog2e = 1.44269504088896340736f;
 
 __device__ __forceinline__ df4 mfma16(dh8 a, dh8 b, df4 c) {
@@ -306,7 +306,7 @@ __global__ __launch_bounds__(64 * W, 2) void attend_decode_kernel(
       for (int a = 0; a < 2; a++)
 #pragma unroll
         for (int i = 0; i < 4; i++) {
-          const float e = __builtin_amdgcn_exp2f(fmaf(s[a][i] - mc, c2, kLift));  // (as in attend_flash.hip)
+          const float e = __builtin_amdgcn_exp2f((s[a][i] - mc) * c2);  // (as in attend_flash.hip)
           p[4 * a + i] = (mine >> (16 * a + i)) & 1 ? e : 0.0f;
           l += p[4 * a + i];
         }
@@ -340,8 +340,8 @@ __global__ __launch_bounds__(64 * W, 2) void attend_decode_kernel(
       if constexpr (!Q8) {
 #pragma unroll
         for (int i = 0; i < 8; i++) {
-          ph[i] = (_Float16)p[i];
-          pl[i] = (_Float16)(p[i] - (float)ph[i]);
+          ph[i] = (_Float16)(p[i] * kLift);
+          pl[i] = (_Float16)fmaf(p[i], kLift, -(float)ph[i]);
         }
       }
 #pragma unroll
@@ -435,7 +435,7 @@ __global__ __launch_bounds__(64 * W, 2) void attend_decode_kernel(
       sum = fmaf(lw[w], f, sum);
     }
     const int64_t slot = slot0 + (int64_t)g * shares;
-    *(df4*)(part_acc + slot * D + d) = v;
+    *(df4*)(part_acc + slot * D + d) = Q8 ? v : v * (1.0f / kLift);
     if (d == 0) *(float2*)(part_ml + slot * 2) = make_float2(m, sum);
   }
 }

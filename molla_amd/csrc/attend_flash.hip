@@ -19,16 +19,18 @@
 //   f32 query, to 2^-39 of its largest value (every bit of values down to 2^-15
 //   of it; two halves left 1e-4 of the output at scores of a few hundred).
 //   O^T = V^T P^T: values lie by rows in LDS and are read transposed
-//   (ds_read_b64_tr_b16); P is lifted by 2^14 and split into two halves (see
-//   kLift).  MFMA step u of a 32-key tile takes keys 8 (i / 4) + 4 h + i % 4
-//   of its 16 in slot (half wave h, i), the order in which S^T leaves them.
+//   (ds_read_b64_tr_b16); P is lifted by 2^14 and split into two halves, each
+//   rounded: to 2^-24 of a weight, as an f32 is (see kLift).  MFMA step u of a
+//   32-key tile takes keys 8 (i / 4) + 4 h + i % 4 of its 16 in slot (half wave
+//   h, i), the order in which S^T leaves them.
 //
 // q8_0: keys enter as their integers (exact halves) and each 32-value
 // block's factor multiplies that block's part of the score; values enter as
 // value * 2^(8 - X) in two halves (7 + 11 bits: exact), X the largest factor's
-// exponent so far in that 32-value block.  A key whose factor is below
-// 2^(X - 22) (its low half would be subnormal) or not finite is left out of the
-// product (its values enter as zeros) and added in float32 at the end, to the
+// exponent so far in that 32-value block; of the four products the one of both
+// low halves is left out, at most 2^-24 of the whole.  A key whose factor is
+// below 2^(X - 22) (its low half would be subnormal) or not finite is left out of
+// the product (its values enter as zeros) and added in float32 at the end, to the
 // rows that it is live for: a later token's factor changes nothing of an earlier
 // one's result.
 //
@@ -61,9 +63,10 @@ typedef uint32_t fu4 __attribute__((ext_vector_type(4)));
 constexpr int kSlice = 64;    // keys a block takes at a time
 constexpr int kRows = 128;    // query rows a block
 // P (at most 1) is lifted by 2^14 before it is split into halves, so that the
-// low halves of weights down to ~1e-8 are not f16 subnormals; the row sums
-// carry the same power of two, which cancels.
-constexpr float kLift = 14.0f;
+// low halves of weights down to ~1e-8 are not f16 subnormals, and the sums are
+// scaled back.  (A lift in the exponential's argument rounds that to 2^-21, weights
+// to 3e-7; the multiplication takes 4 us of a layer's 478 at a chunk of 256.)
+constexpr float kLift = 16384.0f;
 constexpr float kLog2e = 1.44269504088896340736f;
 
 __device__ __forceinline__ ff16 mfma32(fh8 a, fh8 b, ff16 c) {
@@ -403,12 +406,12 @@ __global__ __launch_bounds__(256, 2) void attend_flash_kernel(
     for (int j = 0; j < 16; j++) {
       // (the difference first: at scores of 1e9 c2 mc is rounded by up to 64,
       // and a weight taken against it overflows a half)
-      float p = __builtin_amdgcn_exp2f(fmaf(s[j] - mc, c2, kLift));
+      float p = __builtin_amdgcn_exp2f((s[j] - mc) * c2);
       if (!full) p = live(j) ? p : 0.0f;
       l += p;
-      const _Float16 hi = (_Float16)p;
+      const _Float16 hi = (_Float16)(p * kLift);
       ph[j >> 3][j & 7] = hi;
-      pl[j >> 3][j & 7] = (_Float16)(p - (float)hi);
+      pl[j >> 3][j & 7] = (_Float16)fmaf(p, kLift, -(float)hi);
     }
     if constexpr (Q8) {
 #pragma unroll
@@ -490,7 +493,7 @@ __global__ __launch_bounds__(256, 2) void attend_flash_kernel(
               s = fmaf(__half2float(kfac[st >> 1]), b, s);
             }
             s = other_sum(s);
-            const float p = __builtin_amdgcn_exp2f(fmaf(s - mc, c2, kLift));
+            const float p = __builtin_amdgcn_exp2f((s - mc) * c2) * kLift;
             const float fk = __shfl(f, k) * ldexpf(1.0f, 8 - xo[dt]);
             const int8_t* vb = (const int8_t*)(vc + row) + kvh * D + 32 * dt + 4 * h;
             if (sl * kSlice + k < cnt) {
@@ -508,7 +511,7 @@ __global__ __launch_bounds__(256, 2) void attend_flash_kernel(
   if (!live_row) return;
   const int64_t rowi = (int64_t)t * heads + head;
   float* dst = splits == 1 ? out + rowi * D : part_acc + (rowi * splits + split) * D;
-  const float w = splits == 1 ? 1.0f / l : 1.0f;
+  const float w = (splits == 1 ? 1.0f / l : 1.0f) * (1.0f / kLift);
 #pragma unroll
   for (int dt = 0; dt < NT; dt++) {
     const float f = Q8 ? w * ldexpf(1.0f, xo[dt] - 8) : w;

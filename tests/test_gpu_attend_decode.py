@@ -122,6 +122,41 @@ def test_paged_steps(form, heads, kv, hd, tokens):
 
 
 @pytest.mark.parametrize("form", ["f16", "q8"])
+@pytest.mark.parametrize("hd", [64, 128])
+def test_weights_to_the_last_bits(form, hd):
+    """Two keys with scores 0 and -a and values 0 and 1: the result is the second
+    one's weight, e^-a / (1 + e^-a).  At a up to 1.4 the score's factor and its
+    product with a (2^-24 of at most 2 in base 2), the exponential (an ulp), the
+    sum and the quotient (2^-24) round it: together within 1.1e-7 in the root
+    mean square (6e-8 to 7e-8 is seen).  With P's lift by 2^14 in the exponential's
+    argument, which that rounds to 2^-21, it is 1.4e-7 to 1.5e-7."""
+    from molla_amd import gpu
+    from tests.test_gpu_kernels import q8_rows
+    ctx = gpu.DeviceContext(0)
+    heads, kv = 64, 8
+    kvw = kv * hd
+    k, v = np.zeros((2, kvw), np.float32), np.zeros((2, kvw), np.float32)
+    k[1, ::hd] = -1.0
+    v[1] = 1.0
+    # (a q8_0 factor that is a power of two: 1 / 127 would not be exact)
+    unit = np.float32(127 / 128 if form == "q8" else 1.0)
+    rows = [q8_rows(c * unit, kvw) if form == "q8" else c.astype(np.float16).view(np.uint16).reshape(-1) for c in (k, v)]
+    kd, vd = (torch.from_numpy(r.view(np.int16).copy()).view(torch.float16).cuda() for r in rows)
+    errs = []
+    for seed in range(8):
+        a = np.random.default_rng(seed).uniform(0.05, 1.4, heads).astype(np.float32)
+        q = np.zeros((heads, hd), np.float32)
+        q[:, 0] = a
+        out = torch.zeros(heads * hd, device="cuda")
+        gpu.device_attend(ctx, torch.from_numpy(q.reshape(-1)).cuda(), kd, vd, heads, kv, hd, 1.0, 2, out,
+                          gpu.CACHE_Q8 if form == "q8" else gpu.CACHE_F16)
+        x = a.astype(np.float64) * unit
+        want = np.exp(-x) / (1 + np.exp(-x)) * unit
+        errs.append(out.cpu().numpy().reshape(heads, hd).astype(np.float64) / want[:, None] - 1)
+    assert np.sqrt(np.mean(np.square(errs))) <= 1.1e-7
+
+
+@pytest.mark.parametrize("form", ["f16", "q8"])
 def test_scores_of_1e8(form):
     """Scores whose rounding is worth several powers of two of a weight: the
     largest weight stays 1.  Neighbouring scores lie 1e5 apart and more, so the
