@@ -34,6 +34,32 @@ CASES = [
 @pytest.mark.parametrize("dims,first,tokens", CASES)
 @pytest.mark.parametrize("paged", [False, True])
 def test_chunk_attention_edges(form, dims, first, tokens, paged):
+    against_oracle(form, dims, first, tokens, paged)
+
+
+# (the same), several slices a block
+LONG_CASES = [
+    ((512, 256, 8, 2, 64), 2500, 130),    # 16 shares of 3 slices, the last ones short
+    ((512, 256, 4, 4, 128), 2500, 40),
+    ((512, 256, 8, 1, 128), 3000, 17),
+    ((256, 256, 4, 4, 64), 40, 1000),     # waves of a block end in different slices
+    ((256, 256, 128, 16, 64), 100, 512),  # one share of up to 10 slices: the finished row
+    ((256, 256, 128, 16, 128), 250, 500),
+]
+
+
+@pytest.mark.parametrize("form", ["f16", "q8"])
+@pytest.mark.parametrize("dims,first,tokens", LONG_CASES)
+@pytest.mark.parametrize("paged", [False, True])
+@pytest.mark.parametrize("growing", [False, True])
+def test_chunk_attention_over_several_slices(form, dims, first, tokens, paged, growing):
+    """A block that walks several slices: the buffers' hand-over, the running
+    maximum, and, where the values of every slice are 2^0, 2^7 or 2^-7 of the
+    others' size, the change of the factors' exponent X in a block."""
+    against_oracle(form, dims, first, tokens, paged, growing)
+
+
+def against_oracle(form, dims, first, tokens, paged, growing=False):
     from molla_amd import block, gpu
     from tests.test_gpu_kernels import q8_decode, q8_rows
     ctx = gpu.DeviceContext(0)
@@ -53,6 +79,8 @@ def test_chunk_attention_edges(form, dims, first, tokens, paged):
     kvw, count = bs.kv_width(), first + tokens
     row = gpu.cache_row(f, kvw)
     raw = [synth.normal(count * kvw, 90 + i).numpy().reshape(count, kvw) for i in (0, 1)]
+    if growing:
+        raw[1] *= (2.0 ** (7 * ((np.arange(count) // 64 * 5 + np.arange(count) // 192) % 3 - 1))).astype(np.float32)[:, None]
     rows = [q8_rows(r, kvw).reshape(count, row) if q8 else r.astype(np.float16).view(np.uint16) for r in raw]
     x = synth.normal(tokens * bs.width, 92).numpy()
     xd = torch.from_numpy(x.copy()).cuda()
