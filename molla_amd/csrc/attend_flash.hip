@@ -560,7 +560,8 @@ __global__ __launch_bounds__(256) void attend_combine_kernel(const float* __rest
 }
 
 // Shares of the keys: enough that the blocks fill two a compute unit, at
-// most one for each slice of the context.
+// most one for each slice of the context, and at most 16 (each is another
+// partial result of every row to write and fold).
 int flash_splits(int kv_heads, int tiles, int max_count) {
   const int slices = (max_count + kSlice - 1) / kSlice;
   const int want = 2 * cu_count() / std::max(1, kv_heads * tiles);

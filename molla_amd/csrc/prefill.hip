@@ -277,8 +277,9 @@ struct KB32 {
   // of dwords: they are read from its start, so that on 4-byte aligned weights
   // every load is aligned, and the first block's codes, two bytes off, are
   // moved into place.  (The loads take 2-byte alignment too.  Read at the
-  // codes themselves, half of them two bytes off, Q4_0 4096x14336 at 4 tokens
-  // took 39 us against 27.)
+  // codes themselves, half of them two bytes off, a tile of Q4_0 4096x14336
+  // that held 4 tokens took 39 us against 27; calls of up to 8 tokens take the
+  // kernels of matvec_tile_b32.hip.)
   static constexpr int WORDS = KIND == MI_Q4_0 ? 9 : KIND == MI_Q5_0 ? 11 : KIND == MI_Q8_0 ? 11 : 8 + 2 * (BLOCK - 16) / 4;
   typedef uint32_t v2u_a2 __attribute__((ext_vector_type(2), aligned(2)));
   struct Raw {
@@ -506,12 +507,12 @@ __global__ __launch_bounds__(256) void prefill_prep_kernel(const float* __restri
 // of WR waves over K: group g takes every KS-th 256-value chunk of the block's
 // share, and the groups' sums meet in LDS at the end (no partial sums in
 // memory, where a second launch added them in 10 us at 14336 x 256).
-// What bounds it (14336x4096 Q4_K, 256 tokens, 97 -> 74 us; with the
-// activations' launch and no partial sums 107 -> 88 us a call): 1056 products
-// of 32 cycles a wave, two waves a SIMD, are 28 us at the 2.1 GHz it runs at;
-// half of the products taken out it takes 59 us, the transfer 65, both 53, the
-// decode none: the rest is the LDS reads' latency and the barrier of every
-// stage, with two waves a SIMD to hide them.
+// What bounds it (14336x4096 Q4_K, 256 tokens: 91 -> 71 us; a call, with the
+// activations' launch and no partial sums, 105 -> 79 us): 1056 products of 32
+// cycles a wave, two waves a SIMD, are 32 us at the 2.1 GHz it runs at; half of
+// the products taken out it takes 59 us, the transfer 65, both 53, the decode
+// none: the rest is the LDS reads' latency and the barrier of every stage, with
+// two waves a SIMD to hide them.
 template <int KIND, int RT, int TT, int WR, int KS>
 __global__ __launch_bounds__(WR * KS * 64, (WR * KS + 3) / 4) void prefill_kernel(
     const RowSegs sg, int cols, int tokens, const uint8_t* __restrict__ work, int chunks_per_split,
@@ -791,13 +792,26 @@ struct Shape {
   int rt, tt, wr, ks;
   int block_rows() const { return wr * rt * 32; }
 };
-// Each measured against the others (us, with a split's reduce): up to 32 tokens
-// (1, 1, 4, 2) / (1, 2, 4, 2) / (1, 1, 4, 4): Q4_K 4096x4096 12.7 / 13.8 / 13.5,
-// Q6_K 17.2 / - / 22.9, Q8_0 17.7 / 19.1 / 24.6; Q4_K 6144x4096 at 256 43.7 /
-// 45.7 and 4096x14336 85.0 / 77.3 for (1, 2, 4, 2) / (2, 2, 4, 2): small matrices
-// want more, smaller blocks; Q6_K 4096x14336 at 256 112 / 121 / 135 for
-// (1, 4, 8, 1) / (1, 4, 4, 1) / (2, 2, 4, 2), its three products a step paying for
-// the larger token tile.
+// Each measured against the others (us a call).  Up to 32 tokens (1, 1, 4, 2) /
+// (1, 2, 4, 2) / (1, 1, 4, 4): Q4_K 4096x4096 12.7 / 13.8 / 13.5, Q6_K 17.2 / - /
+// 22.9, Q8_0 17.7 / 19.1 / 24.6.
+// Small matrices want more, smaller blocks.  (1, 2, 4, 2) / (2, 2, 4, 2) by `work`,
+// the 256-value chunks of 256 x 64 outputs:
+//   896   14336x4096, 64 tokens   Q4_K 35.6 / 37.9  Q8_0 44.5 / 47.9  Q4_0 39.0 / 39.3
+//   1232  5632x2048, 400          Q4_K 54.2 / 44.8  Q8_0 59.7 / 61.9  Q4_0 48.8 / 51.2
+//   1536  6144x4096, 256          Q4_K 47.3 / 49.5  Q8_0 65.5 / 66.8  Q4_0 60.5 / 56.0
+//   1792  14336x4096, 128         Q4_K 47.6 / 51.7  Q8_0 68.5 / 72.3  Q4_0 58.1 / 55.8
+//   2064  11008x4096, 192         Q4_K 87.3 / 65.5  Q8_0 107.9 / 105.9  Q4_0 80.5 / 83.2
+//   2688  4096x14336, 192         Q4_K 82.1 / 76.9  Q8_0 122.7 / 116.1  Q4_0 103.2 / 88.8
+//   3584  14336x4096, 256         Q4_K 89.8 / 77.8  Q8_0 111.5 / 113.9  Q4_0 87.7 / 86.4
+// The line is a rough one: the smaller blocks lose where they need a second round
+// of the chip and win up to there (to 2048 for Q4_K and Q8_0), by up to 20 %.
+// Q6_K, three products a step, pays for the larger token tile also where half of
+// it is empty: (1, 2, 4, 2) / (2, 2, 4, 2) / (1, 4, 8, 1) 14336x4096 at 96 tokens
+// 68 / 73 / 62, at 128 69 / 74 / 68, at 150 124 / 117 / 98, 4096x14336 at 192 121 /
+// 120 / 107, at 256 127 / 127 / 114; at 64 48 / 54 / 62.
+// (The (2, 2, 4, 2) block of Q5_1 spills 10 registers in its stage and is still the
+// faster one at 14336x4096, 256 tokens: 118 / 106.)
 Shape shape_for(int kind, int rows, int cols, int tokens) {
   if (tokens <= 32) return Shape{1, 1, 4, 2};
   const int64_t work = (int64_t)((rows + 255) / 256) * ((tokens + 63) / 64) * ((cols + kChunk - 1) / kChunk);
@@ -832,14 +846,14 @@ int launch_kind(hipStream_t s, const RowSegs& sg, int cols, int tokens, const vo
 // Splits of K over blocks (in whole 256-value chunks): the largest power of
 // two whose blocks still fit one round of the chip, one block a compute unit,
 // each K group of a block at least one chunk.
-constexpr int kBlockSlots = 256;
 int choose_splits(int kind, int rows, int cols, int tokens) {
   const Shape sh = shape_for(kind, rows, cols, tokens);
   const int tiles = (tokens + kTileTok - 1) / kTileTok;
   const int64_t blocks = (int64_t)((rows + sh.block_rows() - 1) / sh.block_rows()) * ((tiles + sh.tt - 1) / sh.tt);
   const int chunks = (cols + kChunk - 1) / kChunk;
   int s = 1;
-  while (blocks * 2 * s <= kBlockSlots && chunks >= 2 * s * sh.ks) s *= 2;
+  const int places = cu_count();
+  while (blocks * 2 * s <= places && chunks >= 2 * s * sh.ks) s *= 2;
   return s;
 }
 

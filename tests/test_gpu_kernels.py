@@ -381,16 +381,16 @@ def test_attention(ctx, count):
 
 @pytest.mark.parametrize("count", [5, 300, 2049])
 @pytest.mark.parametrize("heads,kv,hd,qmul", [
-    (32, 8, 128, 1.0),   # groups of 4 (the matrix-core slice kernel)
+    (32, 8, 128, 1.0),   # groups of 4
     (32, 8, 128, 4.0),   # peaky scores: weights down to ~1e-30 in a slice
     (8, 2, 64, 1.0),     # groups of 4, head_dim 64
     (4, 2, 128, 4.0),    # groups of 2
     (2, 2, 64, 1.0),     # groups of 1
-    (16, 2, 128, 1.0),   # groups of 8 (the VALU slice kernel)
+    (16, 2, 128, 1.0),   # groups of 8
 ])
 def test_attention_groups(ctx, count, heads, kv, hd, qmul):
     """f16-cache attention of one token for every query-group size and head
-    width the decode slice kernels take, against the oracle."""
+    width the decode kernels take, against the oracle."""
     from molla_amd import gpu
     kvw = kv * hd
     q = (synth.normal(heads * hd, 31).numpy() * np.float32(qmul)).astype(np.float32)
@@ -436,11 +436,11 @@ def q8_decode(halves, kvw, count):
 @pytest.mark.parametrize("count", [1, 40, 129, 2049])
 @pytest.mark.parametrize("heads,kv,hd", [
     (8, 2, 32),    # the 256-thread slice kernel
-    (8, 2, 64),    # attend_wide_q8_kernel, groups of 4
+    (8, 2, 64),    # attend_decode_kernel, groups of 4
     (8, 2, 128),
     (16, 2, 128),  # groups of 8
     (4, 2, 128),   # groups of 2
-    (2, 2, 64),    # groups of 1: score parts below a 16-byte piece, the slice kernel
+    (2, 2, 64),    # groups of 1
 ])
 def test_attention_q8_cache(ctx, count, heads, kv, hd):
     """tests/test_gpu_ops.mojo test_attend_q8: rows stored by the q8 store

@@ -123,7 +123,7 @@ def test_layer_matches_oracle(dims, pos, tokens, factors):
 def test_batched_config_layer_spread_softmax(tokens):
     """Config 4's shape at 4 and 8 tokens with the attention norm's gain
     scaled by 0.003: q and k elements below one, scores of order one, so
-    the batched attention (the 512-thread slice kernel) and the q|k|v tile's
+    the batched attention (attend_decode_kernel) and the q|k|v tile's
     rope epilogue are checked where the softmax spreads over many keys (with
     N(1, 0.1) gains the scores reach thousands and one key takes all)."""
     _layer_vs_oracle((4096, 14336, 32, 8, 128), 300, tokens, False, attn_gain=0.003)
