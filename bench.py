@@ -68,7 +68,7 @@ def main():
     ap.add_argument("--no-configs", action="store_true", help="skip the BASELINE configs[0] and configs[3] lines")
     args = ap.parse_args()
     if args.gpus != 1:
-        print(f"bench.py measures one GPU: this build has no multi-GPU path (asked for --gpus {args.gpus}).",
+        print(f"bench.py measures one GPU: there is no multi-GPU path (asked for --gpus {args.gpus}).",
               file=sys.stderr)
         sys.exit(2)
 
