@@ -340,7 +340,7 @@ __global__ __launch_bounds__(64 * W, 2) void attend_decode_kernel(
       if constexpr (!Q8) {
 #pragma unroll
         for (int i = 0; i < 8; i++) {
-          ph[i] = (_Float16)(p[i] * kLift);
+          ph[i] = (_Float16)fmaf(p[i], kLift, 0.0f);  // (one instruction)
           pl[i] = (_Float16)fmaf(p[i], kLift, -(float)ph[i]);
         }
       }

@@ -39,10 +39,11 @@
 // 4 (l / 32) + j % 4, column l % 32.
 //
 // What bounds it: 80 MFMA a wave a slice (96 for q8_0; 32 cycles each)
-// against ~1300 cycles of softmax on the VALU, two waves a SIMD.  256 tokens
-// x 32 heads of 128 (8 key heads) behind 3840 positions of f16: 244 us (one
-// block a slice, and its merge) -> 71 us; over 1280 positions of q8_0 (the
-// decode kernel, a token a block) 494 -> 42 us.
+// against ~1300 cycles of softmax on the VALU, two waves a SIMD (the matrix cores
+// are busy a third of the time, the VALU half).  256 tokens x 32 heads of 128 (8
+// key heads) behind 3840 positions of f16: 244 us (one block a slice, and its
+// merge) -> 64 and 9 for the fold; 220 over 1280 positions of q8_0 (the decode
+// kernel, a token a block) 494 -> 41.  At D = 128 it spills 5 to 7 registers.
 #include <math.h>
 
 #include <algorithm>
@@ -65,7 +66,7 @@ constexpr int kRows = 128;    // query rows a block
 // P (at most 1) is lifted by 2^14 before it is split into halves, so that the
 // low halves of weights down to ~1e-8 are not f16 subnormals, and the sums are
 // scaled back.  (A lift in the exponential's argument rounds that to 2^-21, weights
-// to 3e-7; the multiplication takes 4 us of a layer's 478 at a chunk of 256.)
+// to 3e-7; after it, it takes 2 us of a layer's 470 at a chunk of 256.)
 constexpr float kLift = 16384.0f;
 constexpr float kLog2e = 1.44269504088896340736f;
 
@@ -409,7 +410,7 @@ __global__ __launch_bounds__(256, 2) void attend_flash_kernel(
       float p = __builtin_amdgcn_exp2f((s[j] - mc) * c2);
       if (!full) p = live(j) ? p : 0.0f;
       l += p;
-      const _Float16 hi = (_Float16)(p * kLift);
+      const _Float16 hi = (_Float16)fmaf(p, kLift, 0.0f);  // (one instruction)
       ph[j >> 3][j & 7] = hi;
       pl[j >> 3][j & 7] = (_Float16)fmaf(p, kLift, -(float)hi);
     }
