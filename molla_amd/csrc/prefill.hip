@@ -805,7 +805,7 @@ struct Shape {
 //   2688  4096x14336, 192         Q4_K 82.1 / 76.9  Q8_0 122.7 / 116.1  Q4_0 103.2 / 88.8
 //   3584  14336x4096, 256         Q4_K 89.8 / 77.8  Q8_0 111.5 / 113.9  Q4_0 87.7 / 86.4
 // The line is a rough one: the smaller blocks lose where they need a second round
-// of the chip and win up to there (to 2048 for Q4_K and Q8_0), by up to 20 %.
+// of the chip (up to 25 %) and for Q4_K and Q8_0 win up to there, to 2048 (11 %).
 // Q6_K, three products a step, pays for the larger token tile also where half of
 // it is empty: (1, 2, 4, 2) / (2, 2, 4, 2) / (1, 4, 8, 1) 14336x4096 at 96 tokens
 // 68 / 73 / 62, at 128 69 / 74 / 68, at 150 124 / 117 / 98, 4096x14336 at 192 121 /
