@@ -457,10 +457,12 @@ bool decode_attend_fits(int32_t group, int32_t head_dim) {
 // the blocks run side by side or in turn, and about a quarter of a run's for each
 // block (us as above; 2304 keys, 18 steps, 32 pairs of a token and a key head: 6
 // shares of 3 are 192 blocks and 46.1, 9 of 2 are 288 and 49.3, 18 of 1 are 576 and
-// 46.9; 64 pairs: 4 shares 64.6, 6 64.8, 8 66.3, 16 69.9).  Of the equal ones the
-// fewest.  q8_0's loads wait on more arithmetic, so that one block a unit is a
-// sixteenth slower than that (eight paged sequences of 6000: 4 shares 87.4, 8 82.0,
-// 16 87.0).  At most 64, which the fold takes in one round.
+// 46.9; 64 pairs: 4 shares 64.6, 6 64.8, 8 66.3, 16 69.9).  The fold takes another
+// 1/128 of a run's for each share (one q8_0 sequence of 9000 in a context of 16384:
+// 32 shares 35.2, 64 38.0).  q8_0's loads wait on more arithmetic, so that one block
+// a unit is a little slower than that (eight paged sequences of 6000: 4 shares 86.3,
+// 8 78.7, 16 83.0; two of 9000: 16 shares 52.8, 32 54.2).  At most 64 shares, which
+// the fold takes in one round.
 DecodePlan decode_attend_plan(int32_t kv_heads, int32_t tokens, int32_t max_count, bool q8) {
   const int64_t pairs = (int64_t)kv_heads * tokens, cus = cu_count();
   const int waves = pairs * ((max_count - 1) / (2 * kRun) + 1) <= cus ? 2 : 4;
@@ -469,8 +471,8 @@ DecodePlan decode_attend_plan(int32_t kv_heads, int32_t tokens, int32_t max_coun
   int64_t least = INT64_MAX;
   for (int n = 1; n <= std::min<int64_t>(steps, kMaxShares); n++) {
     const int64_t deep = (n * pairs + cus - 1) / cus;
-    int64_t cost = 16 * deep * (4 * ((steps + n - 1) / n) + 1);
-    if (q8 && deep == 1) cost += cost / 16;
+    int64_t cost = 16 * deep * (4 * ((steps + n - 1) / n) + 1) + n / 2;
+    if (q8 && deep == 1) cost += cost / 32;
     if (cost < least) best.shares = n, least = cost;
   }
   return best;
