@@ -10,17 +10,17 @@
 // (no block barrier until the waves' results are folded at the end), and sends for
 // the next run's keys and values as soon as it has used this one's.  The number of
 // shares (decode_attend_plan) is the one with the fewest runs in line on a compute
-// unit and stays at 64, so a long context costs a few partial results a head and
+// unit, at most 64, so a long context costs a few partial results a head and
 // not one a 64-key slice.
 //
-// What bounds it: to about 1000 keys a chain of latencies (of ~7500 cycles of a
-// block with one run a wave the position takes ~1000, the keys ~2500, the softmax
-// ~800, the weighted values ~700, the fold ~1000); beyond, the loads: a layer's
-// attention over 32768 keys f16, cold, moves 134 MB in 34 us.  us of a layer of
-// width 256 with 32 heads of 128 over 8 key heads, caches cold (a 64-key slice a
-// block and a merge of the slices -> now): one sequence of 300 keys 26.2 -> 26.4, of
-// 2304 28.6 -> 28.3, of 32768 71.2 -> 51.1; eight of 300 50.9 -> 50.5, of 2304 64.7 ->
-// 64.6, of 8000 102.7 -> 96.4; eight of 6000 and less, paged q8_0, 101.5 -> 79.5.
+// What bounds it: to about 1000 keys a chain of latencies (cycles of a block with
+// one run a wave: the position ~1000, the keys ~2500, the softmax ~800, the values
+// to LDS ~400, the weighted values ~700, then the fold); beyond, the loads.  us of
+// a layer of width 256 with 32 heads of 128 over 8 key heads, caches cold (a 64-key
+// slice a block and a merge of the slices -> now): one sequence of 300 keys 26.2 ->
+// 26.4, of 2304 28.6 -> 28.3, of 32768 71.2 -> 51.1; eight of 300 50.9 -> 50.5, of
+// 2304 64.7 -> 64.6, of 8000 102.7 -> 96.4; eight of 6000 and less, paged q8_0, 101.5
+// -> 79.5.
 //
 //   S^T = K Q^T, keys as rows (read straight from the cache) and queries as
 //   columns: a lane's 8 scores belong to its own query, the softmax takes two
@@ -111,7 +111,7 @@ __global__ __launch_bounds__(64 * W, 2) void attend_decode_kernel(
   constexpr int KS = D / 32, NT = D / 16, PIECES = D / 8;
   constexpr int kFac = Q8 ? 2 * KS * kRun : 1;             // floats: factors of a run's keys and values
   constexpr int kWaveBytes = kRun * D * 2;                 // a run's values as halves
-  __shared__ __align__(16) uint8_t vs[W][kWaveBytes];  // afterwards the waves' sums
+  __shared__ __align__(16) uint8_t vs[W][kWaveBytes];      // afterwards the waves' sums
   __shared__ __align__(16) float fac[W][kFac];
   __shared__ __align__(16) float wml[2][8][W];  // (maximum, sum) of a head, the waves side by side
   static_assert(8 * D * 4 <= kWaveBytes, "a wave's sums of 8 heads in place of its values");
